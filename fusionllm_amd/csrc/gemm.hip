@@ -29,6 +29,7 @@
 // small_gemm_kernel, which streams the weights once (when no group of the
 // launch can exceed 2 kSmallM rows, every group, in slabs of kSmallM).
 #include <atomic>
+#include <type_traits>
 
 #include "fmoe_common.h"
 #include "gemm_core.h"
@@ -82,53 +83,52 @@ struct GemmArgs {
 // rows past N are clamped to the last valid one (their products are never
 // stored), so no operand is read out of bounds.
 
-// Tile t -> (group g, m tile tm, n tile tn, first row, group rows); false if t
-// is past the last tile.
-// offsets: args.offsets passed as a separate restrict pointer, so that these
-// uniform reads become scalar loads (a vector load would need a vmcnt wait that
-// also waits for the in-flight operand copies).
-__device__ __forceinline__ bool locate_tile(const GemmArgs& a, const int32_t* __restrict__ offsets, int tiles_n,
-                                            int t, int& g, int& tm, int& tn, int& row_base, int& M) {
-  const int G = a.E + (a.rows_shared > 0 ? 1 : 0);
-  for (g = 0; g < G; ++g) {
-    if (g < a.E) {
-      const int2 o = core::sload2(offsets + g);
-      row_base = o.x;
-      M = o.y - o.x;
-    } else {
-      row_base = a.rows_routed;
-      M = a.rows_shared;
-    }
-    const int nt = (M <= a.small_max) ? 0 : ((M + core::BM - 1) / core::BM) * tiles_n;
-    if (t < nt) {
-      tm = t / tiles_n;
-      tn = t - tm * tiles_n;
-      return true;
-    }
-    t -= nt;
-  }
-  return false;
+// Tile -> (group, rows) map of a launch, held by the lanes of each wave: lane
+// e < E has expert e's first row, rows and first tile, so that a tile is found
+// with one ballot and three lane reads.  (A walk over the groups with a scalar
+// load each took 2-3 us per tile at E = 64, twice per tile: in the copy cursor
+// and in the epilogue.)
+struct TileMap {
+  int row, rows, start;  // of expert `lane` (start: INT_MAX past the last expert)
+  int routed, total;     // tiles of the routed groups, of all groups
+};
+
+struct Tile {
+  int g, tm, tn, row_base, M;  // group, m tile, n tile, the group's first row and rows
+};
+
+__device__ __forceinline__ TileMap tile_map(const GemmArgs& a, const int32_t* __restrict__ offsets, int tiles_n,
+                                            int lane) {
+  TileMap m;
+  const int lo = offsets[min(lane, a.E)], hi = offsets[min(lane + 1, a.E)];
+  m.row = lo;
+  m.rows = hi - lo;  // 0 past the last expert
+  const int nt = (m.rows <= a.small_max) ? 0 : ((m.rows + core::BM - 1) / core::BM) * tiles_n;
+  const int incl = wave_incl_scan(nt, lane);
+  m.start = lane < a.E ? incl - nt : INT32_MAX;
+  m.routed = __builtin_amdgcn_readlane(incl, 63);
+  m.total = m.routed + ((a.rows_shared <= a.small_max) ? 0 : ((a.rows_shared + core::BM - 1) / core::BM) * tiles_n);
+  return m;
 }
 
-__device__ __forceinline__ int count_tiles(const GemmArgs& a, const int32_t* __restrict__ offsets, int tiles_n) {
-  const int G = a.E + (a.rows_shared > 0 ? 1 : 0);
-  int total = 0;
-  for (int g = 0; g < G; ++g) {
-    int M = a.rows_shared;
-    if (g < a.E) {
-      const int2 o = core::sload2(offsets + g);
-      M = o.y - o.x;
-    }
-    total += (M <= a.small_max) ? 0 : ((M + core::BM - 1) / core::BM) * tiles_n;
+// Tile t < total: the last expert whose first tile is at most t (experts
+// without tiles start where the next one does, or past t).
+__device__ __forceinline__ Tile locate_tile(const GemmArgs& a, const TileMap& m, int tiles_n, int t) {
+  Tile r;
+  if (t >= m.routed) {
+    r.g = a.E;
+    r.row_base = a.rows_routed;
+    r.M = a.rows_shared;
+    t -= m.routed;
+  } else {
+    r.g = 63 - __builtin_clzll(__ballot(m.start <= t));
+    r.row_base = __builtin_amdgcn_readlane(m.row, r.g);
+    r.M = __builtin_amdgcn_readlane(m.rows, r.g);
+    t -= __builtin_amdgcn_readlane(m.start, r.g);
   }
-  return total;
-}
-
-// Store instructions per lane in the epilogue of a full tile (they may still
-// be in flight at the next barrier; see the wait there).
-template <int MODE>
-constexpr int epi_stores() {
-  return MODE == GATEUP_FWD ? 24 : (MODE == DOWN_BWD ? 32 : 16);
+  r.tm = t / tiles_n;
+  r.tn = t - r.tm * tiles_n;
+  return r;
 }
 
 // K-split of the last, partial round of tiles.  With T tiles on P
@@ -245,12 +245,10 @@ __device__ __forceinline__ void swiglu_bwd8(const uint4& dhv, const uint4& av, c
 // the block has accumulators, so the block is first staged whole: dh rounded
 // to bf16, through the wave's 4 KB of LDS one 16-row slice at a time, read
 // back as 16-byte row segments (64 registers, the accumulators are then
-// free).  The a|b loads then run as a pipeline two slices deep (the loads of
-// slice i + 2 issued while slice i is computed and stored); a deeper one
-// measured no faster.  Row pointers are uniform (scalar registers); a lane
-// adds one offset.  Measured at C2 against the previous slice-by-slice
-// epilogue (a|b of one slice in flight while it was staged): 266-279 ->
-// 258-265 us, bit-identical.
+// free); then the slices' a|b are loaded, computed and stored one after
+// another.  Row pointers are uniform (scalar registers); a lane adds one
+// offset.  Two slices of loads in flight spill 51 registers beside the main
+// loop's (C2 302 against 260 us, C5 1855 against 1510 us).
 __device__ __forceinline__ void down_bwd_full_epilogue(const GemmArgs& args, const f32x4 (&acc)[core::FM][core::FN],
                                                        uint8_t* ep, int el, int64_t grow0, int col0) {
   using namespace core;
@@ -282,26 +280,20 @@ __device__ __forceinline__ void down_bwd_full_epilogue(const GemmArgs& args, con
   const uint32_t coff = static_cast<uint32_t>((el >> 4) * static_cast<int>(args.ldc0) + (el & 15) * 8) * 2u;
   const int64_t cstep = args.ldc0 * 2 * 4;
   const int64_t binter = args.inter * 2;  // bytes from a to b (and from da to db)
-  constexpr int kDepth = 2;               // slices of a|b loads in flight
-  uint4 pa[FM][4], pb[FM][4];
-  auto load_slice = [&](int i) {
+  asm volatile("" ::: "memory");  // the loads are not hoisted into the staging above
+#pragma unroll
+  for (int i = 0; i < FM; ++i) {
+    uint4 pa[4], pb[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       const uint8_t* rp = abase + (i * 4 + t) * astep;
-      pa[i][t] = load16(reinterpret_cast<const uint16_t*>(rp + aoff), true);
-      pb[i][t] = load16(reinterpret_cast<const uint16_t*>(rp + binter + aoff), true);
+      pa[t] = load16(reinterpret_cast<const uint16_t*>(rp + aoff), true);
+      pb[t] = load16(reinterpret_cast<const uint16_t*>(rp + binter + aoff), true);
     }
-  };
-  asm volatile("" ::: "memory");  // the loads are not hoisted into the staging above
-#pragma unroll
-  for (int i = 0; i < kDepth; ++i) load_slice(i);
-#pragma unroll
-  for (int i = 0; i < FM; ++i) {
-    if (i > 0 && i + kDepth - 1 < FM) load_slice(i + kDepth - 1);
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       uint4 dav, dbv;
-      swiglu_bwd8(dhv[i][t], pa[i][t], pb[i][t], dav, dbv);
+      swiglu_bwd8(dhv[i][t], pa[t], pb[t], dav, dbv);
       uint8_t* rp = cbase + (i * 4 + t) * cstep;
       store16(reinterpret_cast<uint16_t*>(rp + coff), dav, true);
       store16(reinterpret_cast<uint16_t*>(rp + binter + coff), dbv, true);
@@ -328,7 +320,8 @@ __global__ __launch_bounds__(core::NT, 1) void rows_gemm_kernel(const GemmArgs a
   // transposing LDS reads.
   constexpr bool BTR = (MODE == DOWN_BWD || MODE == GATEUP_BWD);
   const int tiles_n = (args.N + TN_COLS - 1) / TN_COLS;
-  const int total_tiles = count_tiles(args, offsets, tiles_n);
+  const TileMap map = tile_map(args, offsets, tiles_n, lane);
+  const int total_tiles = map.total;
   const int NP = static_cast<int>(gridDim.x), b = xcd_slot(static_cast<int>(blockIdx.x), NP);
   const int nk = args.K / BK;
   const SplitPlan sp = split_plan<MODE>(args, total_tiles, NP, nk);
@@ -336,189 +329,183 @@ __global__ __launch_bounds__(core::NT, 1) void rows_gemm_kernel(const GemmArgs a
     // descriptors of the split tiles for the split reduction (after the
     // partials): first row, valid rows, first output column, valid columns
     // (GATEUP_FWD: h columns, 128 per tile)
-    if (args.split_ws != nullptr && threadIdx.x == 0) {
+    const int r = static_cast<int>(blockIdx.x);
+    if (args.split_ws != nullptr) {
       int4* hdr = reinterpret_cast<int4*>(args.split_ws + static_cast<int64_t>(NP) * BM * BN);
-      const int r = static_cast<int>(blockIdx.x);
-      if (r == 0) hdr[0] = make_int4(sp.R, sp.S, 0, 0);
+      if (r == 0 && threadIdx.x == 0) hdr[0] = make_int4(sp.R, sp.S, 0, 0);
       if (r < sp.R) {
-        int g, tm, tn, row_base, M;
-        locate_tile(args, offsets, tiles_n, sp.full + r, g, tm, tn, row_base, M);
-        hdr[1 + r] = make_int4(row_base + tm * BM, min(M - tm * BM, BM), tn * TN_COLS,
-                               min(args.N - tn * TN_COLS, TN_COLS));
+        const Tile t = locate_tile(args, map, tiles_n, sp.full + r);
+        if (threadIdx.x == 0)
+          hdr[1 + r] = make_int4(t.row_base + t.tm * BM, min(t.M - t.tm * BM, BM), t.tn * TN_COLS,
+                                 min(args.N - t.tn * TN_COLS, TN_COLS));
       }
     }
   }
   const int my_items = (sp.items() - b + NP - 1) / NP;  // items b, b + NP, ...
   if (my_items <= 0) return;
-  int total = 0;  // K steps of 64 over all of this workgroup's items
-  for (int i = 0; i < my_items; ++i) {
+  // K steps of 64 over all of this workgroup's items (only the last can be a range)
+  int total = (my_items - 1) * nk;
+  {
     int t_, k0_, kn_, s_;
-    split_item(sp, nk, b + i * NP, t_, k0_, kn_, s_);
+    split_item(sp, nk, b + (my_items - 1) * NP, t_, k0_, kn_, s_);
     total += kn_;
   }
 
   // ---- global -> LDS copy cursor
-  // Copy instruction i of wave w writes LDS rows 64 i + 8 w .. +7 of an operand;
-  // lane l fetches row 64 i + drow, global chunk dchunk (the swizzled slot l % 8).
-  const int drow = w * 8 + (lane >> 3);
-  const int dchunk = (lane & 7) ^ swzk(drow);  // swzk(64 i + drow) == swzk(drow)
-  // B as it lies (BTR): k row 16 i + drow_b, chunk cb_t (wsw(16 i + drow_b) == wsw(drow_b))
-  const int drow_b = 2 * w + (lane >> 5);
-  const int cb_t = ((((lane & 31) >> 1) ^ wsw(drow_b)) << 1) | (lane & 1);
-  const uint32_t lds_copy = sbase + w * 1024;
-  int c_ti = 0, c_kt = 0, c_k0 = 0, c_kn = 0;  // item ordinal, step within it, its K range
-  const uint16_t* c_a = nullptr;   // A rows of the tile being copied
-  const uint16_t* c_b0 = nullptr;  // B operand base(s)
-  const uint16_t* c_b1 = nullptr;
-  int c_last_row = 0, c_n0 = 0;    // last valid A row of the tile, first B row
-  // GA: this lane's byte offsets (from c_a) of its A rows of the tile, rows
-  // 64 i + drow clamped to the last valid one; the routed rows are token rows
-  // of x (row r: x row gather[r] / gather_k).  The lane's four indices of an
-  // item are loaded when the item before it is set up (g_pf, vector loads
-  // issued after that stage's copies, complete by the next stage's wait) and
-  // consumed one item later.
-  uint32_t a_off[LA];
-  int32_t g_pf[LA] = {0, 0, 0, 0};
-  bool g_pf_routed = false;  // the prefetched item is a routed tile (its rows are gathered)
-  auto item_rows = [&](int ti, int& row0, int& last, bool& routed) {
-    int tile, k0_, kn_, slot;
-    split_item(sp, nk, b + ti * NP, tile, k0_, kn_, slot);
-    int g, tm, tn, row_base, M;
-    routed = locate_tile(args, offsets, tiles_n, tile, g, tm, tn, row_base, M) && g < args.E;
-    row0 = row_base + tm * BM;
-    last = min(M - tm * BM, BM) - 1;
-  };
-  auto prefetch_rows = [&](int ti) {
-    // item ti's indices (no loads past the last item or for the shared group)
-    g_pf_routed = false;
-    if (ti >= my_items) return;
-    int row0, last;
-    item_rows(ti, row0, last, g_pf_routed);
-    if (!g_pf_routed) return;
-#pragma unroll
-    for (int i = 0; i < LA; ++i) {
-      const uint32_t off = static_cast<uint32_t>(row0 + min(64 * i + drow, last)) * 4u;
-      asm volatile("global_load_dword %0, %1, %2" : "+v"(g_pf[i]) : "v"(off), "s"(args.gather) : "memory");
-    }
-  };
-  auto copy_tile = [&](int ti) {
-    int tile, slot;
-    split_item(sp, nk, b + ti * NP, tile, c_k0, c_kn, slot);
-    int g, tm, tn, row_base, M;
-    locate_tile(args, offsets, tiles_n, tile, g, tm, tn, row_base, M);
-    const bool gathered = GA && g < args.E;
-    const uint16_t* A = gathered ? args.a_routed
-                        : (g < args.E || args.a_shared == nullptr) ? args.a_routed + static_cast<int64_t>(row_base) * args.lda
-                                                                   : args.a_shared;
-    c_a = gathered ? A : A + static_cast<int64_t>(tm) * BM * args.lda;
-    c_last_row = min(M - tm * BM, BM) - 1;
-    c_b0 = args.b0[g];
-    c_b1 = args.b1[g];
-    c_n0 = tn * TN_COLS;
-    if constexpr (GA) {
-      if (gathered) {
-        // g_pf holds this item's indices (loaded one item ahead, a stage wait
-        // has normally passed since; the wait here covers every operation older
-        // than this stage's LT copies and orders the use after it)
-        asm volatile("s_waitcnt vmcnt(%4)"
-                     : "+v"(g_pf[0]), "+v"(g_pf[1]), "+v"(g_pf[2]), "+v"(g_pf[3])
-                     : "n"(LT)
-                     : "memory");
-#pragma unroll
-        for (int i = 0; i < LA; ++i) {
-          const uint32_t tok = slot_token(static_cast<uint32_t>(g_pf[i]), args.gather_magic);
-          a_off[i] = (tok * static_cast<uint32_t>(args.lda) + static_cast<uint32_t>(dchunk * 8)) * 2u;
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < LA; ++i)
-          a_off[i] = static_cast<uint32_t>(min(64 * i + drow, c_last_row) * static_cast<int>(args.lda) + dchunk * 8) * 2u;
-      }
-      prefetch_rows(ti + 1);
-    }
-  };
-  if constexpr (GA) {
-    // the first item's indices, waited for at once
-    prefetch_rows(0);
-    asm volatile("s_waitcnt vmcnt(0)" : "+v"(g_pf[0]), "+v"(g_pf[1]), "+v"(g_pf[2]), "+v"(g_pf[3])::"memory");
-  }
-  copy_tile(0);
+  // A stage is copied in halves of four instructions: half u holds rows 32 u ..
+  // +31 of every wave's 64 A rows and rows (columns of the output) 64 u .. +63
+  // of every wave's 128 B rows.  Instruction i of wave w writes eight LDS rows,
+  // lane l fetches row l / 8 of them, global chunk dchunk (the swizzled slot
+  // l % 8).
+  const uint32_t lds_a = sbase + (64 * (w >> 2) + 8 * (w & 3)) * RB;
+  const uint32_t lds_b = sbase + A_BYTES + w * 1024;
+  int c_ti = 0, c_kt = 0, c_kn = 0;  // item ordinal, step within it, its steps
+  const uint8_t* c_a = nullptr;      // A rows of the tile being copied, at the step's k
+  const uint8_t* c_b0 = nullptr;     // B operand(s), at the step's k
+  const uint8_t* c_b1 = nullptr;
+  int c_ksw = 0;                     // GATEUP_BWD: the step at which B goes on in w3
+  // this lane's byte offsets from c_a / c_b* of the tile (rows and columns past
+  // the end clamped to the last valid one), formed once per tile; [2 u + i]
+  constexpr int NBO = (MODE == GATEUP_FWD) ? 2 : 4;
+  uint32_t a_off[4], b_off[NBO];
   const int lda = static_cast<int>(args.lda), ldb = static_cast<int>(args.ldb);
-  auto issue = [&](int it) {
-    const uint32_t st = lds_copy + (it & 1) * STAGE;
-    const int kofs = (c_k0 + c_kt) * BK;
-    auto copy_a = [&]() {
-#pragma unroll
-      for (int i = 0; i < LA; ++i) {
-        if constexpr (GA) {
-          copy16(st + i * 8192, c_a + kofs, a_off[i]);
-        } else {
-          const int r = min(64 * i + drow, c_last_row);
-          copy16(st + i * 8192, c_a + kofs, static_cast<uint32_t>(r * lda + dchunk * 8) * 2u);
-        }
-      }
-    };
-    auto copy_b = [&]() {
-      if constexpr (BTR) {
-        // 64 k rows of 512 bytes: instruction i of wave w writes k rows 16 i + 2 w, +1;
-        // lane l: k row 16 i + drow_b, logical 16-byte chunk cb_t (32-byte windows
-        // swizzled by wsw(k row)).  GATEUP_BWD: k < inter from w1, else from w3.
-        const uint16_t* bb = (MODE == GATEUP_BWD && kofs >= args.inter)
-                                 ? c_b1 + static_cast<int64_t>(kofs - args.inter) * args.ldb
-                                 : c_b0 + static_cast<int64_t>(kofs) * args.ldb;
-        const int col = min(c_n0 + 8 * cb_t, args.N - 8);
-#pragma unroll
-        for (int i = 0; i < LB; ++i)
-          copy16(st + A_BYTES + i * 8192, bb, static_cast<uint32_t>((16 * i + drow_b) * ldb + col) * 2u);
-      } else {
-#pragma unroll
-        for (int i = 0; i < LB; ++i) {
-          // GATEUP_FWD bands: w1 rows (even i) and w3 rows (odd i), 64 h columns each
-          const int n = min(c_n0 + ((MODE == GATEUP_FWD) ? (i >> 1) * 64 : 64 * i) + drow, args.N - 1);
-          const uint16_t* b = (MODE == GATEUP_FWD && (i & 1)) ? c_b1 : c_b0;
-          copy16(st + A_BYTES + i * 8192, b + kofs, static_cast<uint32_t>(n * ldb + dchunk * 8) * 2u);
-        }
-      }
-    };
-    // The dX products issue the weight rows first (512-byte rows of a matrix
-    // that every CU streams) and the activation rows after them: gate/up dX
-    // 289 -> 283 us at C2, the down backward within noise; in the forward
-    // products the order made no difference (same instructions and waits).
+  auto copy_tile = [&](int ti) __attribute__((always_inline)) {
+    int tile, slot, k0;
+    split_item(sp, nk, b + ti * NP, tile, k0, c_kn, slot);
+    const Tile t = locate_tile(args, map, tiles_n, tile);
+    const bool gathered = GA && t.g < args.E;
+    const uint16_t* A = gathered ? args.a_routed
+                        : (t.g < args.E || args.a_shared == nullptr)
+                            ? args.a_routed + static_cast<int64_t>(t.row_base) * args.lda
+                            : args.a_shared;
+    if (!gathered) A += static_cast<int64_t>(t.tm) * BM * args.lda;
+    c_a = reinterpret_cast<const uint8_t*>(A + k0 * BK);
+    const int last_row = min(t.M - t.tm * BM, BM) - 1, n0 = t.tn * TN_COLS;
+    // the lane as an opaque value: what follows is formed here, not kept in
+    // registers through the main loop
+    int l = lane;
+    asm volatile("" : "+v"(l));
+    const int dchunk = (l & 7) ^ swzk(l >> 3);
     if constexpr (BTR) {
-      copy_b();
-      copy_a();
+      // B as it lies: unit u holds columns 64 u .. +63 of every wave's 128;
+      // instruction i of wave w writes its k rows 32 i + krow, 16-byte chunk
+      // cb of a row (wsw(32 i + krow) == wsw(krow))
+      const int krow = 4 * w + (l >> 4);
+      const int cb = ((((l & 15) >> 1) ^ wsw(krow)) << 1) | (l & 1);
+      const int col = 128 * (cb >> 3) + 8 * (cb & 7);  // + 64 u: its column of the tile
+      // GATEUP_BWD: k < inter from w1, else from w3
+      const int kb = k0 * BK;
+      const bool hi = MODE == GATEUP_BWD && kb >= args.inter;
+      c_b0 = reinterpret_cast<const uint8_t*>((hi ? args.b1[t.g] : args.b0[t.g]) +
+                                              static_cast<int64_t>(hi ? kb - args.inter : kb) * args.ldb);
+      c_b1 = reinterpret_cast<const uint8_t*>(args.b1[t.g]);
+      c_ksw = hi ? INT32_MAX : args.inter / BK - k0;
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        b_off[q] = static_cast<uint32_t>((32 * (q & 1) + krow) * ldb + min(n0 + 64 * (q >> 1) + col, args.N - 8)) * 2u;
     } else {
-      copy_a();
-      copy_b();
+      c_b0 = reinterpret_cast<const uint8_t*>(args.b0[t.g] + k0 * BK);
+      if constexpr (MODE == GATEUP_FWD) c_b1 = reinterpret_cast<const uint8_t*>(args.b1[t.g] + k0 * BK);
+      // GATEUP_FWD: the wave's first 64 B rows are w1 rows, the others the w3 rows of the same h columns
+#pragma unroll
+      for (int q = 0; q < NBO; ++q) {
+        const int n = min(n0 + ((MODE == GATEUP_FWD) ? 64 * q : 128 * (q & 1) + 64 * (q >> 1)) + 8 * w + (l >> 3), args.N - 1);
+        b_off[q] = static_cast<uint32_t>(n * ldb + dchunk * 8) * 2u;
+      }
     }
-    if (++c_kt == c_kn) {
-      c_kt = 0;
-      if (++c_ti < my_items) copy_tile(c_ti);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int r = min(64 * (w >> 2) + 8 * (w & 3) + (l >> 3) + 128 * (q & 1) + 32 * (q >> 1), last_row);
+      // gathered: the routed rows are token rows of x, row r: x row gather[r] / gather_k
+      // (the index loads are waited for here, once per tile)
+      if (gathered) {
+        const uint32_t slot = static_cast<uint32_t>(args.gather[t.row_base + t.tm * BM + r]);
+        a_off[q] = (slot_token(slot, args.gather_magic) * static_cast<uint32_t>(lda) + static_cast<uint32_t>(dchunk * 8)) * 2u;
+      } else {
+        a_off[q] = static_cast<uint32_t>(r * lda + dchunk * 8) * 2u;
+      }
+    }
+  };
+  copy_tile(0);
+  // Unit u of step it's stage (two instructions): a stage's units are issued
+  // in the order A0, B0, B1, A1, and A1 moves the cursor on.  Past the last
+  // step the last stage is copied again (into slots that are free and not read
+  // any more), so that every wait counts the same operations.
+  auto issue_a = [&](int it, int u) __attribute__((always_inline)) {
+    const uint32_t st = lds_a + (it & 1) * STAGE;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) copy16(st + (128 * i + 32 * u) * RB, c_a, a_off[2 * u + i]);
+    if (u == 0) return;
+    const int64_t bstep = BTR ? 2 * BK * args.ldb : RB;
+    c_a += RB;
+    c_b0 += bstep;
+    if constexpr (MODE == GATEUP_FWD) c_b1 += RB;
+    if (__builtin_expect(++c_kt == c_kn, 0)) {
+      if (c_ti + 1 < my_items) {
+        c_kt = 0;
+        copy_tile(++c_ti);
+      } else {  // past the end: the last stage again
+        --c_kt;
+        c_a -= RB;
+        c_b0 -= bstep;
+        if constexpr (MODE == GATEUP_FWD) c_b1 -= RB;
+      }
+    } else if (MODE == GATEUP_BWD && c_kt == c_ksw) {
+      c_b0 = c_b1;  // (a range that ends at the last row of w1 never gets here)
+    }
+  };
+  auto issue_b = [&](int it, int u) __attribute__((always_inline)) {
+    const uint32_t st = lds_b + (it & 1) * STAGE;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      if constexpr (BTR)
+        copy16(st + u * UNIT + i * 8192, c_b0, b_off[2 * u + i]);
+      else if constexpr (MODE == GATEUP_FWD)
+        copy16(st + (128 * i + 64 * u) * RB, u ? c_b1 : c_b0, b_off[i]);
+      else
+        copy16(st + (128 * i + 64 * u) * RB, c_b0, b_off[2 * u + i]);
     }
   };
 
-  // ---- fragment address bases (A rows / B rows of this wave; BTR: trb_base)
+  // ---- fragments: A rows 16 f of the wave's 64 (units a0, a1: f 0..1, 2..3),
+  // B rows 16 f of its 128 (b0, b1: f 0..3, 4..7)
   uint32_t xa = frag_base(wm * WTM, lane);
-  uint32_t xb = BTR ? trb_base(wn, lane) : frag_base(wn * WTN, lane);
+  uint32_t xb = A_BYTES + (BTR ? tr_base(4 * wn, lane) : frag_base(wn * WTN, lane));
+  AFrag a0, a1;
+  BFrag b0, b1;
+  typedef __attribute__((address_space(3))) bf16x8 lds_bf16x8;
+  auto lds_frag = [&](uint32_t x, uint32_t src, int kh, int f) {
+    return *(const lds_bf16x8*)(uintptr_t)((x ^ (kh * 64u)) + src + 2048u * f);
+  };
+  auto read_a = [&](AFrag& f, int u, uint32_t src, int kh, int m) { f[kh][m] = lds_frag(xa, src, kh, 2 * u + m); };
+  auto read_b = [&](BFrag& f, int u, uint32_t src, int kh, int n) {
+    if constexpr (BTR)
+      f[kh][n] = tr_frag(((src + xb) ^ (n << 5)) + u * UNIT + kh * TR_KHALF);
+    else
+      f[kh][n] = lds_frag(xb, src, kh, 4 * u + n);
+  };
 
-  issue(0);
-  if (total > 1) {
-    issue(1);
-    wait_vm_barrier<LT>();
-  } else {
-    wait_vm_barrier<0>();
-  }
-  bf16x8 P[FN], Q[2][4];
+  // The fragments a tile starts with: A0 whole, B0's first 32-deep half.
+  auto read_first = [&](uint32_t src) {
 #pragma unroll
-  for (int p = 0; p < FN; ++p)
-    P[p] = BTR ? trb_frag(sbase + (xb ^ (static_cast<uint32_t>(p) << 5)))
-               : *reinterpret_cast<const bf16x8*>(smem + A_BYTES + (xb + 2048u * p));
+    for (int kh = 0; kh < 2; ++kh)
 #pragma unroll
-  for (int q = 0; q < 4; ++q) Q[0][q] = *reinterpret_cast<const bf16x8*>(smem + (xa + 2048u * q));
-  // Q[1] is a read-write operand of the first block8 statements (overwritten
-  // there by their ds_reads): give it a defined value.
+      for (int m = 0; m < 2; ++m) read_a(a0, 0, src, kh, m);
 #pragma unroll
-  for (int q = 0; q < 4; ++q) Q[1][q] = Q[0][q];
+    for (int n = 0; n < 4; ++n) read_b(b0, 0, src, 0, n);
+  };
+
+  issue_a(0, 0);
+  issue_b(0, 0);
+  issue_b(0, 1);
+  issue_a(0, 1);
+  issue_a(1, 0);
+  issue_b(1, 0);
+  issue_b(1, 1);
+  wait_vm_barrier<5 * LU>();
+  read_first(sbase);
+  const bool late = w >= 4;  // this wave's SIMD partner is one phase ahead
+  if (late) barrier();
 
   f32x4 acc[FM][FN];
 #pragma unroll
@@ -532,35 +519,45 @@ __global__ __launch_bounds__(core::NT, 1) void rows_gemm_kernel(const GemmArgs a
     int k0_;
     split_item(sp, nk, b, e_tile, k0_, e_kn, e_slot);
   }
-  int last_epi = -4;        // iteration whose end wrote an epilogue
-  bool last_full = false;   // that epilogue issued exactly epi_stores<MODE>() stores
+  // At a step's waits, only the units issued after the ones waited for may be
+  // in flight (counting the stores of the last epilogue as well, so that they
+  // need not have completed, measured no faster and takes branches).
   for (int it = 0; it < total; ++it) {
     // keep the per-step fragment addresses from being hoisted out of the loop
     asm volatile("" : "+v"(xa), "+v"(xb));
-    const uint32_t cur = sbase + (it & 1) * STAGE;
-    if constexpr (BTR)
-      kstep_t<1>(acc, P, Q[0], Q[1], xa, xb, cur);
-    else
-      kstep<64>(acc, P, Q[0], Q[1], xa, xb, cur);  // reads the second K half of this stage
-    uint32_t src = cur;                           // the last step re-reads (harmlessly) its own stage
-    if (it + 1 < total) {
-      // Stage (it+1) must have landed; stage it&1 is free once every wave is past
-      // this point.  Stores of an epilogue written after copy it+1 was issued may
-      // still be in flight (only when their number is exact).
-      if (it - last_epi == 1 && last_full)
-        wait_vm_barrier<epi_stores<MODE>()>();
-      else
-        wait_vm_barrier<0>();
-      if (it + 2 < total) issue(it + 2);
-      src = sbase + ((it + 1) & 1) * STAGE;
-    }
-    if constexpr (BTR)
-      kstep_t<0>(acc, P, Q[1], Q[0], xa, xb, src);
-    else
-      kstep<0>(acc, P, Q[1], Q[0], xa, xb, src);
+    const uint32_t cur = sbase + (it & 1) * STAGE, nxt = sbase + ((it + 1) & 1) * STAGE;
+    // (0, 0)
+#pragma unroll
+    for (int n = 0; n < 4; ++n) read_b(b0, 0, cur, 1, n);
+    issue_a(it + 1, 1);
+    wait_vm_barrier<5 * LU>();  // B1 of this stage
+    quarter<0, 0>(acc, a0, b0);
+    // (0, 1)
+#pragma unroll
+    for (int kh = 0; kh < 2; ++kh)
+#pragma unroll
+      for (int n = 0; n < 4; ++n) read_b(b1, 1, cur, kh, n);
+    issue_a(it + 2, 0);
+    wait_vm_barrier<5 * LU>();  // A1 of this stage
+    quarter<0, 1>(acc, a0, b1);
+    // (1, 0)
+#pragma unroll
+    for (int kh = 0; kh < 2; ++kh)
+#pragma unroll
+      for (int m = 0; m < 2; ++m) read_a(a1, 1, cur, kh, m);
+    issue_b(it + 2, 0);
+    wait_vm_barrier<4 * LU>();  // A0, B0 of the next stage
+    quarter<1, 0>(acc, a1, b0);
+    // (1, 1): the next step's first fragments (at a tile's end they are read
+    // again after its epilogue, which needs the registers)
+    read_first(nxt);
+    issue_b(it + 2, 1);
+    wait_lds_barrier();
+    quarter<1, 1>(acc, a1, b1);
 
     if (++e_kt < e_kn) continue;
-    // ---- tile epilogue: this wave's 64 x 128 block
+    // ---- tile epilogue: this wave's 64 x 128 block (both wave groups together)
+    if (!late) barrier();
     e_kt = 0;
     asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3\n" ::: "memory");  // MFMA results -> VALU reads
     // lane index as an opaque value: keeps the epilogue's address arithmetic
@@ -577,12 +574,11 @@ __global__ __launch_bounds__(core::NT, 1) void rows_gemm_kernel(const GemmArgs a
           *reinterpret_cast<f32x4*>(part + (wm * WTM + i * 16 + (el & 15)) * BN + wn * WTN + j * 16 + (el >> 4) * 4) =
               acc[i][j];
     } else {
-      int g, tm, tn, row_base, M;
-      locate_tile(args, offsets, tiles_n, e_tile, g, tm, tn, row_base, M);
-      const int rows_valid = min(M - tm * BM, BM);
-      const int col0 = tn * TN_COLS + wn * (TN_COLS / WN);  // first output column of this wave
-      const bool full = rows_valid == BM && (tn + 1) * TN_COLS <= args.N;
-      const int64_t grow0 = static_cast<int64_t>(row_base) + tm * BM + wm * WTM;
+      const Tile t = locate_tile(args, map, tiles_n, e_tile);
+      const int rows_valid = min(t.M - t.tm * BM, BM);
+      const int col0 = t.tn * TN_COLS + wn * (TN_COLS / WN);  // first output column of this wave
+      const bool full = rows_valid == BM && (t.tn + 1) * TN_COLS <= args.N;
+      const int64_t grow0 = static_cast<int64_t>(t.row_base) + t.tm * BM + wm * WTM;
       bool epi_done = false;
       if constexpr (MODE == DOWN_BWD) {
         if (full) {
@@ -687,34 +683,22 @@ __global__ __launch_bounds__(core::NT, 1) void rows_gemm_kernel(const GemmArgs a
           }
         }
       }
-      last_full = full;
     }  // whole tile
-    if (e_slot >= 0) last_full = false;
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
       for (int j = 0; j < FN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     asm volatile("s_nop 1" ::: "memory");  // VALU writes -> MFMA reads of the accumulators
-    last_epi = it;
-    if constexpr (MODE == DOWN_BWD) {
-      // The fragments the last K step read for the next tile are read again
-      // (its first stage has landed, waited for above; after the last tile
-      // the reads harmlessly re-read a stage), so that their registers are
-      // free during the epilogue, which needs them for the a|b loads (no
-      // branch in the K loop: a K step that skipped the reads before an
-      // epilogue kept both sets live and spilled).
-      const uint32_t nst = sbase + ((it + 1) & 1) * STAGE;
-      typedef __attribute__((address_space(3))) bf16x8 lds_bf16x8;
-#pragma unroll
-      for (int p = 0; p < FN; ++p) P[p] = trb_frag(nst + (xb ^ (static_cast<uint32_t>(p) << 5)));
-#pragma unroll
-      for (int q = 0; q < 4; ++q) Q[0][q] = *(const lds_bf16x8*)(uintptr_t)(nst + xa + 2048u * q);
-    }
+    // the next tile's first fragments (after the last tile a harmless re-read)
+    read_first(sbase + ((it + 1) & 1) * STAGE);
+    if (late && it + 1 < total) barrier();
     if (++e_ti < my_items) {
       int k0_;
       split_item(sp, nk, b + e_ti * NP, e_tile, k0_, e_kn, e_slot);
     }
   }
+  // the copies past the end have landed before the workgroup's LDS is given back
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
 // ---- split reductions
@@ -1130,16 +1114,6 @@ __device__ __forceinline__ void group_rows(const WgradArgs& a, int g, int& row_b
 // column 4 q): two such reads give a lane 8 consecutive k of one output row.
 // The 32-byte windows of a k row are XOR-swizzled by wsw(row) so that the 16
 // rows x 32 bytes a read instruction touches fall on distinct banks.
-using core::wsw;
-
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ bf16x8 tr_frag(uint32_t addr) {
-  typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-  const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(uintptr_t)addr);
-  const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(uintptr_t)(addr + 2048u));
-  return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-}
-
 // GATHER: args.b_gather is set (a separate instantiation, so that the plain
 // kernel carries none of the gathered path's code).
 template <bool GATHER>
@@ -1148,9 +1122,10 @@ __global__ __launch_bounds__(core::NT, 1) void wgrad_tr_kernel(const WgradArgs a
   using namespace core;
   __shared__ __attribute__((aligned(1024))) uint8_t smem[2 * STAGE];
   // Gathered B rows: the slot indices of each stage's 64 k rows (ring of eight
-  // stages, filled by global -> LDS copies three stages ahead and read one
-  // stage ahead, after the stage waits that cover them; a slot is refilled
-  // four stages after its last read, with stage barriers in between).
+  // stages, filled by global -> LDS copies three stages ahead of a stage's
+  // copies and read when its first B unit is issued, after waits that cover
+  // them; a slot is refilled stages after its last read, with barriers in
+  // between).
   __shared__ int32_t idx_ring[8][BK];
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1217,155 +1192,181 @@ __global__ __launch_bounds__(core::NT, 1) void wgrad_tr_kernel(const WgradArgs a
       copy4(ring + (kt & 7) * (BK * 4), args.b_gather + row_base, static_cast<uint32_t>(r) * 4u);
     }
   };
-  // ---- copies: instruction i of wave w writes k rows 16 i + drow (1 KB = 2 rows of 512 B);
-  // lane chunk p = l % 32 holds logical chunk c of the row
-  const int drow = 2 * w + (lane >> 5);
-  const int p = lane & 31;
-  const int c = (((p >> 1) ^ wsw(drow)) << 1) | (p & 1);  // wsw(16 i + drow) == wsw(drow)
-  const int colA = min(m0 + 8 * c, args.m_out - 8), colB = min(n0 + 8 * c, args.n_out - 8);
+  // ---- copies: a unit is 128 columns of a stage's 64 k rows (A0, A1, B0, B1
+  // in LDS); instruction i of wave w writes its k rows 32 i + drow (1 KB = 4
+  // rows of 256 B), lane chunk p = l % 16 holds logical chunk c of the row
+  const int drow = 4 * w + (lane >> 4);
+  const int p = lane & 15;
+  const int c = (((p >> 1) ^ wsw(drow)) << 1) | (p & 1);  // wsw(32 i + drow) == wsw(drow)
   const uint32_t lds_copy = sbase + w * 1024;
-  uint32_t b_off[4];  // gathered B: this lane's byte offsets (from B) of its 4 k rows of a coming stage
-  auto form_offsets = [&](int kt) {
-    const int last = k_end - 1 - (k_begin + kt * BK);  // >= 0 for kt < nk
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = min(16 * i + drow, last);
-      const uint32_t tok = slot_token(static_cast<uint32_t>(idx_ring[kt & 7][r]), args.gather_magic);
-      b_off[i] = (tok * static_cast<uint32_t>(ldb) + static_cast<uint32_t>(colB)) * 2u;
-    }
-  };
   if (gathered) {
-    // stages 0..2 before the first copies (issue(kt) fetches stage kt + 3)
+    // stages 0..2 before the first copies (stage kt's last unit fetches stage kt + 3)
     for (int q = 0; q < 3 && q < nk; ++q) fetch_idx(q);
     asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
   }
 
-  auto issue = [&](int kt) {
-    const int k0 = k_begin + kt * BK;
-    const int last = k_end - 1 - k0;  // last valid k row of this stage
-    const uint32_t st = lds_copy + (kt & 1) * STAGE;
+  // Unit u of a stage (two instructions); a stage's units are issued in the
+  // order A0, B0, B1, A1, and A1 moves on to the next stage.  Past the last
+  // stage the last one is copied again (into slots that are free and not read
+  // any more), so that every wait counts the same operations.
+  // The lane's byte offsets from the stage's first rows (pa, pb): columns past
+  // the end clamped to the last ones, rows past k_end to the last valid row
+  // (only the last stage can have some).
+  const uint8_t* pa = reinterpret_cast<const uint8_t*>(A + static_cast<int64_t>(k_begin) * lda);
+  const uint8_t* pb = reinterpret_cast<const uint8_t*>(gathered ? B : B + static_cast<int64_t>(k_begin) * ldb);
+  uint32_t a_off[4], b_off[4];  // [2 u + i]
+  auto form_rows = [&](int kt) {
+    const int last = k_end - 1 - (k_begin + kt * BK);  // >= 0 for kt < nk
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = min(16 * i + drow, last);
-      copy16(st + i * 8192, A + static_cast<int64_t>(k0) * lda, static_cast<uint32_t>(r * lda + colA) * 2u);
+    for (int q = 0; q < 4; ++q) {
+      const int r = min(32 * (q & 1) + drow, last);
+      a_off[q] = static_cast<uint32_t>(r * lda + min(m0 + 128 * (q >> 1) + 8 * c, args.m_out - 8)) * 2u;
+      if (!gathered) b_off[q] = static_cast<uint32_t>(r * ldb + min(n0 + 128 * (q >> 1) + 8 * c, args.n_out - 8)) * 2u;
     }
-    if (gathered) {
-      // k row r of the stage is x row (slot of group row k0 + r) / k, at the
-      // offsets b_off formed from the stage's ring slot (at the end of the K
-      // step before, or before the first copies)
+  };
+  // gathered B: k row r of a stage is x row (slot of group row k0 + r) / k, from
+  // the stage's ring slot
+  auto form_gathered = [&](int kt) {
+    const int last = k_end - 1 - (k_begin + kt * BK);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) copy16(st + A_BYTES + i * 8192, B, b_off[i]);
-      if (kt + 3 < nk) fetch_idx(kt + 3);
-    } else {
+    for (int i = 0; i < 2; ++i) {
+      const int r = min(32 * i + drow, last);
+      const uint32_t tok = slot_token(static_cast<uint32_t>(idx_ring[kt & 7][r]), args.gather_magic);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int r = min(16 * i + drow, last);
-        copy16(st + A_BYTES + i * 8192, B + static_cast<int64_t>(k0) * ldb,
-               static_cast<uint32_t>(r * ldb + colB) * 2u);
-      }
+      for (int u = 0; u < 2; ++u)
+        b_off[2 * u + i] = (tok * static_cast<uint32_t>(ldb) +
+                            static_cast<uint32_t>(min(n0 + 128 * u + 8 * c, args.n_out - 8))) * 2u;
     }
+  };
+  form_rows(0);
+  auto issue_a = [&](int kt, int u) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) copy16(lds_copy + (kt & 1) * STAGE + u * UNIT + i * 8192, pa, a_off[2 * u + i]);
+    if (u == 0) return;
+    if (GATHER && gathered && kt + 3 < nk) fetch_idx(kt + 3);
+    if (kt + 1 < nk) {
+      pa += 2 * BK * args.lda;
+      if (!gathered) pb += 2 * BK * args.ldb;
+      if (kt + 2 == nk) form_rows(kt + 1);
+    }
+  };
+  auto issue_b = [&](int kt, int u) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      copy16(lds_copy + (kt & 1) * STAGE + A_BYTES + u * UNIT + i * 8192, pb, b_off[2 * u + i]);
   };
   // Rows past k_end in a stage hold copies of the last valid row: zero their A
   // side (after this wave's copies have landed) so that they add nothing.
-  auto zero_tail = [&](int kt) {
+  auto zero_tail = [&](int kt, int u) {
     const int k0 = k_begin + kt * BK;
-    if (k_end - k0 >= BK) return;
-    uint8_t* st = smem + (kt & 1) * STAGE + w * 1024 + lane * 16;
+    if (kt >= nk || k_end - k0 >= BK) return;
+    uint8_t* st = smem + (kt & 1) * STAGE + u * UNIT + w * 1024 + lane * 16;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (k0 + 16 * i + drow >= k_end) *reinterpret_cast<uint4*>(st + i * 8192) = make_uint4(0, 0, 0, 0);
+    for (int i = 0; i < 2; ++i)
+      if (k0 + 32 * i + drow >= k_end) *reinterpret_cast<uint4*>(st + i * 8192) = make_uint4(0, 0, 0, 0);
   };
-  auto sync_stage = [&](int kt, bool more_in_flight) {
-    if (more_in_flight) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    zero_tail(kt);
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  // All but the N newest copies of this wave have landed (the gathered rows'
+  // index fetches make wave 0's count differ, so that variant waits for all).
+  auto wait_copies = [&](auto n) {
+    if (GATHER) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(decltype(n)::value) : "memory");
   };
 
-  // ---- fragment addresses: lane (h, s = 4 jq + q); window swizzle fr = wsw(8 h + jq)
-  const int h = lane >> 4, jq = (lane >> 2) & 3, q = lane & 3;
-  const int fr = jq | ((h & 1) << 2);
-  const uint32_t xa = static_cast<uint32_t>((8 * h + jq) * 512 + (((4 * wm) ^ fr) << 5) + 8 * q);
-  const uint32_t xb = static_cast<uint32_t>(A_BYTES + (8 * h + jq) * 512 + ((8 * wn + fr) << 5) + 8 * q);
+  // ---- fragment addresses within a unit: the wave's 32 A columns (2 windows), 64 B columns (4)
+  uint32_t xa = tr_base(2 * wm, lane), xb = A_BYTES + tr_base(4 * wn, lane);
+  AFrag a0, a1;
+  BFrag b0, b1;
+  auto read_a = [&](AFrag& f, uint32_t unit, int kh, int m) { f[kh][m] = tr_frag(((unit + xa) ^ (m << 5)) + kh * TR_KHALF); };
+  auto read_b = [&](BFrag& f, uint32_t unit, int kh, int n) { f[kh][n] = tr_frag(((unit + xb) ^ (n << 5)) + kh * TR_KHALF); };
+  auto read_first = [&](uint32_t src) {
+#pragma unroll
+    for (int kh = 0; kh < 2; ++kh)
+#pragma unroll
+      for (int m = 0; m < 2; ++m) read_a(a0, src, kh, m);
+#pragma unroll
+    for (int n = 0; n < 4; ++n) read_b(b0, src, 0, n);
+  };
 
-  if (gathered) form_offsets(0);
-  issue(0);
-  if (nk > 1) {
-    if (gathered) form_offsets(1);
-    issue(1);
-  }
-  if (gathered) form_offsets(min(2, nk - 1));
-  sync_stage(0, nk > 1);
+  if (gathered) form_gathered(0);
+  issue_a(0, 0);
+  issue_b(0, 0);
+  issue_b(0, 1);
+  issue_a(0, 1);
+  if (gathered) form_gathered(min(1, nk - 1));
+  issue_a(1, 0);
+  issue_b(1, 0);
+  issue_b(1, 1);
+  wait_copies(std::integral_constant<int, 5 * LU>{});
+  zero_tail(0, 0);
+  wait_lds_barrier();
 
   f32x4 acc[FM][FN];
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  bf16x8 fa[FM], fb[FN];
-#pragma unroll
-  for (int f = 0; f < FM; ++f) fa[f] = tr_frag(sbase + (xa ^ (f << 5)));
-#pragma unroll
-  for (int f = 0; f < FN; ++f) fb[f] = tr_frag(sbase + (xb ^ (f << 5)));
+  asm volatile("s_nop 1" ::: "memory");  // VALU writes -> MFMA reads of the accumulators
+  read_first(sbase);
+  const bool late = w >= 4;
+  if (late) barrier();
 
   for (int kt = 0; kt < nk; ++kt) {
-    const uint32_t cur = sbase + (kt & 1) * STAGE;
+    asm volatile("" : "+v"(xa), "+v"(xb));
+    const uint32_t cur = sbase + (kt & 1) * STAGE, nxt = sbase + ((kt + 1) & 1) * STAGE;
+    // (0, 0)
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      uint32_t src = cur + 16384u;  // second K half of this stage
-      if (ks == 1) {
-        src = cur;  // the last step re-reads (harmlessly) its own stage
-        if (kt + 1 < nk) {
-          sync_stage(kt + 1, false);
-          if (kt + 2 < nk) issue(kt + 2);
-          src = sbase + ((kt + 1) & 1) * STAGE;
-        }
-      }
-      bf16x8 na[FM], nb[FN];
+    for (int n = 0; n < 4; ++n) read_b(b0, cur, 1, n);
+    issue_a(kt + 1, 1);
+    wait_copies(std::integral_constant<int, 5 * LU>{});  // B1 of this stage
+    wait_lds_barrier();
+    quarter<0, 0>(acc, a0, b0);
+    // (0, 1)
 #pragma unroll
-      for (int f = 0; f < FM; ++f) na[f] = tr_frag(src + (xa ^ (f << 5)));
+    for (int kh = 0; kh < 2; ++kh)
 #pragma unroll
-      for (int f = 0; f < FN; ++f) nb[f] = tr_frag(src + (xb ^ (f << 5)));
+      for (int n = 0; n < 4; ++n) read_b(b1, cur + UNIT, kh, n);
+    issue_a(kt + 2, 0);
+    wait_copies(std::integral_constant<int, 5 * LU>{});  // A1 of this stage
+    zero_tail(kt, 1);
+    wait_lds_barrier();
+    quarter<0, 1>(acc, a0, b1);
+    // (1, 0)
 #pragma unroll
-      for (int i = 0; i < FM; ++i)
+    for (int kh = 0; kh < 2; ++kh)
 #pragma unroll
-        for (int j = 0; j < FN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[j], fa[i], acc[i][j], 0, 0, 0);
-      // interleave: per 8 MFMAs, 6 fragment reads (24 reads, 32 MFMAs per step)
-#pragma unroll
-      for (int x = 0; x < 4; ++x) {
-        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-        __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-        __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-      }
-#pragma unroll
-      for (int f = 0; f < FM; ++f) fa[f] = na[f];
-#pragma unroll
-      for (int f = 0; f < FN; ++f) fb[f] = nb[f];
-    }
-    // gathered B: the offsets of stage kt + 3 (issued in the next K step),
-    // formed after this step's MFMAs rather than right after a barrier,
-    // where every wave would wait for its ring reads at once.  The ring slot
-    // landed before this step's second wait; past the last stage the last
-    // one is formed again (unused).
-    if (gathered) form_offsets(min(kt + 3, nk - 1));
+      for (int m = 0; m < 2; ++m) read_a(a1, cur + UNIT, kh, m);
+    // gathered B: the offsets of stage kt + 2, whose ring slot landed a step ago
+    if (gathered) form_gathered(min(kt + 2, nk - 1));
+    issue_b(kt + 2, 0);
+    wait_copies(std::integral_constant<int, 4 * LU>{});  // A0, B0 of the next stage
+    zero_tail(kt + 1, 0);
+    wait_lds_barrier();
+    quarter<1, 0>(acc, a1, b0);
+    // (1, 1)
+    read_first(nxt);  // past the last stage: a harmless read
+    issue_b(kt + 2, 1);
+    wait_lds_barrier();
+    quarter<1, 1>(acc, a1, b1);
   }
+  if (!late) barrier();
+  asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3\n" ::: "memory");  // MFMA results -> VALU reads
+  // the copies past the end have landed before the workgroup's LDS is given back
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
-  // ---- epilogue: lane holds C[m0 + 64 wm + 16 i + l % 16][n0 + 128 wn + 16 j + 4 (l / 16) + 0..3]
+  // ---- epilogue: lane holds C[m0 + 128 (i / 2) + 32 wm + 16 (i % 2) + l % 16]
+  //                           [n0 + 128 (j / 4) + 64 wn + 16 (j % 4) + 4 (l / 16) + 0..3]
   const int64_t mn = static_cast<int64_t>(args.m_out) * args.n_out;
   float* part = (chunks > 1) ? args.partial + static_cast<int64_t>(pbase + chunk) * mn : nullptr;
 #pragma unroll
   for (int i = 0; i < FM; ++i) {
-    const int m = m0 + wm * WTM + i * 16 + (lane & 15);
+    const int m = m0 + (i >> 1) * 128 + wm * 32 + (i & 1) * 16 + (lane & 15);
     if (m >= args.m_out) continue;
     const bool lo = m < args.m_split;
     void* base = lo ? args.out_lo[g] : args.out_hi[g];
     const int64_t orow = static_cast<int64_t>(lo ? m : m - args.m_split) * args.n_out;
 #pragma unroll
     for (int j = 0; j < FN; ++j) {
-      const int n = n0 + wn * WTN + j * 16 + (lane >> 4) * 4;
+      const int n = n0 + (j >> 2) * 128 + wn * 64 + (j & 3) * 16 + (lane >> 4) * 4;
       if (n >= args.n_out) continue;
       const f32x4 v = acc[i][j];
       if (part) {

@@ -3,20 +3,36 @@
 //
 // Tile: 256 x 256 outputs per 512-thread workgroup (8 waves, 4 x 2, each wave a
 // 64 x 128 sub-tile of 4 x 8 blocks of v_mfma_f32_16x16x32_bf16), K stepped by
-// 64 through two LDS stages of 64 KB (operand rows of 128 bytes, K-contiguous).
+// 64 through two LDS stages of 64 KB.
 //
 // * Global -> LDS copies use global_load_lds_dwordx4 (16 bytes per lane written
-//   straight into LDS, no VGPR round trip).  One wave instruction writes 1 KB
-//   of LDS = 8 rows; the 16-byte chunks of a row are XOR-swizzled
-//   (slot = chunk ^ (row & 7), swzk below) by choosing which global chunk a
-//   lane fetches, which makes the fragment reads below free of bank conflicts.
-// * The copies and the LDS fragment reads are issued from inline assembly so
-//   that the compiler neither reorders them nor inserts conservative
-//   vmcnt(0) waits between the copies and the reads; every wait is explicit.
-// * 32-deep K steps are split into four blocks of 8 MFMAs.  Each block reads,
-//   interleaved with its MFMAs, the fragments that the same block of the next
-//   step needs: the eight B-side fragments ("P") are reloaded in place right
-//   after their last use, the four A-side fragments ("Q") are double buffered.
+//   straight into LDS, no VGPR round trip), issued from inline assembly so that
+//   the compiler neither reorders them nor waits for them: every wait on them
+//   is explicit.  Operands whose rows are K-contiguous (128-byte rows in LDS)
+//   have the 16-byte chunks of a row XOR-swizzled (slot = chunk ^ (row & 7),
+//   swzk below) by choosing which global chunk a lane fetches, which makes the
+//   fragment reads free of bank conflicts.
+// * A stage is four 16 KB units A0, A1, B0, B1: half of each wave's rows (A)
+//   and columns (B), with all 64 k.  A K step is four quarters of a wave's
+//   block, (A0, B0), (A0, B1), (A1, B0), (A1, B1), 16 MFMAs each.  A unit is in
+//   registers a quarter or two after it was first read, and its slot is then
+//   refilled with the stage after the next: five to six units (80 - 96 KB) are
+//   in flight at any time, against 64 KB for half of the time when a whole
+//   stage was consumed before its slot was refilled.
+// * Every quarter is a read phase (its LDS reads, two copies, a wait) and an
+//   MFMA phase, each ended by a workgroup barrier.  Waves 4 - 7 run one phase
+//   behind waves 0 - 3, so the two waves of a SIMD alternate: one issues MFMAs
+//   while the other reads and copies.  The phases hold no branches (past the
+//   last step the copies repeat the last stage instead of stopping; stores of
+//   an epilogue are waited for like the copies): a few scalar instructions
+//   more in each read phase cost 10-25 % of the loop.
+//   Measured on MI355X, cycles of a 64-deep step (2048 at the MFMA rate): 3270
+//   with one barrier and eight copies per step, both waves of a SIMD in step;
+//   2200 - 2580 in this form (a whole chip on random data then runs at 1.6 -
+//   1.8 GHz, power-limited).  C2 (49152 rows, d = 768, I = 2048): gate/up
+//   forward 355 -> 305 us, down forward 178 -> 148, gate/up dX 304 -> 277; C5
+//   (262144 rows, d = 2048, I = 1408): 2770 -> 2140, 1490 -> 1045, 2560 -> 2140;
+//   outputs bit-identical.
 // * MFMA operands are swapped (srcA = B fragment, srcB = A fragment), so that a
 //   lane's 4 accumulators hold 4 consecutive output columns of one row:
 //   acc[i][j] of lane l = C[16 i + l % 16][16 j + 4 (l / 16) + 0..3].
@@ -36,7 +52,10 @@ constexpr int SMEM = 2 * STAGE + 8 * EPI;   // 160 KB: the whole LDS of a CU
 constexpr int WM = 4, WN = 2;               // wave grid
 constexpr int WTM = BM / WM, WTN = BN / WN; // 64 x 128 per wave
 constexpr int FM = WTM / 16, FN = WTN / 16; // 4 x 8 blocks of 16 x 16
-constexpr int LA = 4, LB = 4, LT = LA + LB; // copy instructions per lane per stage
+constexpr int LT = 8;                       // copy instructions per lane per stage
+constexpr int LU = LT / 4;                  // ... per unit
+constexpr int UNIT = 16384;                 // bytes of a unit (half of an operand's stage)
+constexpr int UNIT_ROW = 256;               // bytes of a k row of a unit copied as it lies (128 columns)
 
 // Operand stages: 16-byte chunk c of 128-byte row r sits at slot c ^ swzk(r).
 // With this swizzle the fragment reads below (lane l: row l % 16 of a
@@ -70,19 +89,13 @@ __device__ __forceinline__ int2 sload2(const int32_t* p) {
   return v;
 }
 
-// Scalar load of eight consecutive ints at a wave-uniform address (tracked by
-// lgkmcnt, waited for at once, as sload2).
-typedef int i32x8 __attribute__((ext_vector_type(8)));
-__device__ __forceinline__ i32x8 sload8(const int32_t* p) {
-  i32x8 v;
-  asm volatile("s_load_dwordx8 %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)\n" : "=s"(v) : "s"(p) : "memory");
-  return v;
-}
-
 // One 4-byte-per-lane copy global -> LDS (lane l writes LDS bytes lds + 4 l).
 __device__ __forceinline__ void copy4(uint32_t lds, const void* base, uint32_t voff) {
   asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2\n" ::"s"(lds), "v"(voff), "s"(base) : "memory");
 }
+
+// Workgroup barrier (no waits).
+__device__ __forceinline__ void barrier() { asm volatile("s_barrier" ::: "memory"); }
 
 // Wait until at most N vector-memory operations of this wave are in flight and
 // its LDS reads are done, then synchronise the workgroup.
@@ -91,41 +104,8 @@ __device__ __forceinline__ void wait_vm_barrier() {
   static_assert(N >= 0 && N < 64, "vmcnt range");
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier\n" ::"n"(N) : "memory");
 }
-
-#define FMOE_MF(c, a, b) "v_mfma_f32_16x16x32_bf16 " c ", " a ", " b ", " c "\n"
-#define FMOE_DS(d, p) "ds_read_b128 " d ", " p "\n"
-
-// Block x of a 32-deep K step: acc[q][2x + p] += A_q (x) B_(2x+p) for q = 0..3,
-// p = 0..1.  Reads next-step fragments: Q'[x] (A side) into nq, and P[2x],
-// P[2x+1] (B side) in place after their last use.  WAIT = lgkmcnt bound that
-// guarantees the fragments this block consumes have arrived.
-// The reads are still in flight when the statement ends: their destinations
-// are read-write operands ("+v"), so each keeps one register across the loop
-// that is consumed only by a later block8, after the s_waitcnt that covers
-// it (tests/test_host.py checks the built code for any other access to a
-// pending ds_read destination).
-template <int WAIT>
-__device__ __forceinline__ void block8(f32x4& c00, f32x4& c01, f32x4& c02, f32x4& c03, f32x4& c10, f32x4& c11,
-                                       f32x4& c12, f32x4& c13, bf16x8& p0, bf16x8& p1, const bf16x8& q0,
-                                       const bf16x8& q1, const bf16x8& q2, const bf16x8& q3, bf16x8& nq,
-                                       uint32_t aq, uint32_t ap0, uint32_t ap1) {
-  asm volatile(
-      "s_waitcnt lgkmcnt(%[wt])\n"
-      FMOE_DS("%[nq]", "%[aq]")
-      FMOE_MF("%[c00]", "%[p0]", "%[q0]") FMOE_MF("%[c01]", "%[p0]", "%[q1]")
-      FMOE_MF("%[c02]", "%[p0]", "%[q2]") FMOE_MF("%[c03]", "%[p0]", "%[q3]")
-      FMOE_DS("%[p0]", "%[ap0]")
-      FMOE_MF("%[c10]", "%[p1]", "%[q0]") FMOE_MF("%[c11]", "%[p1]", "%[q1]")
-      FMOE_MF("%[c12]", "%[p1]", "%[q2]") FMOE_MF("%[c13]", "%[p1]", "%[q3]")
-      FMOE_DS("%[p1]", "%[ap1]")
-      : [c00] "+v"(c00), [c01] "+v"(c01), [c02] "+v"(c02), [c03] "+v"(c03), [c10] "+v"(c10), [c11] "+v"(c11),
-        [c12] "+v"(c12), [c13] "+v"(c13), [p0] "+v"(p0), [p1] "+v"(p1), [nq] "+v"(nq)
-      : [q0] "v"(q0), [q1] "v"(q1), [q2] "v"(q2), [q3] "v"(q3), [aq] "v"(aq), [ap0] "v"(ap0), [ap1] "v"(ap1),
-        [wt] "n"(WAIT));
-}
-
-#undef FMOE_MF
-#undef FMOE_DS
+// The same, waiting for the LDS reads only.
+__device__ __forceinline__ void wait_lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier\n" ::: "memory"); }
 
 // LDS address of fragment f of one operand: the lane's row (16 f + l % 16 of
 // the wave's block) at chunk (l / 16 + 4 * step half), swizzled.  For rows
@@ -141,102 +121,71 @@ __device__ __forceinline__ uint32_t frag_addr(uint32_t x, uint32_t src) {
   return (x ^ static_cast<uint32_t>(KX)) + (src + 2048u * F);
 }
 
-// One 32-deep K step of the wave's 64 x 128 sub-tile on fragments P (B side,
-// 8) and Qc (A side, 4), reading the next step's fragments (Qn, P in place)
-// from the stage at LDS address src, K half KX (0 or 64).  xa / xb: frag_base
-// of the wave's A rows and B rows (B rows offset by A_BYTES in src).
-template <int KX>
-__device__ __forceinline__ void kstep(f32x4 (&acc)[FM][FN], bf16x8 (&P)[FN], bf16x8 (&Qc)[4], bf16x8 (&Qn)[4],
-                                      uint32_t xa, uint32_t xb, uint32_t src) {
-  const uint32_t srcb = src + A_BYTES;
-  // Block 0 needs Q'[3] of the previous step (two reads younger): lgkmcnt(2);
-  // block x > 0 needs P[2x], P[2x+1] of the previous step (nine reads younger).
-  block8<2>(acc[0][0], acc[1][0], acc[2][0], acc[3][0], acc[0][1], acc[1][1], acc[2][1], acc[3][1], P[0], P[1],
-            Qc[0], Qc[1], Qc[2], Qc[3], Qn[0], frag_addr<0, KX>(xa, src), frag_addr<0, KX>(xb, srcb),
-            frag_addr<1, KX>(xb, srcb));
-  block8<9>(acc[0][2], acc[1][2], acc[2][2], acc[3][2], acc[0][3], acc[1][3], acc[2][3], acc[3][3], P[2], P[3],
-            Qc[0], Qc[1], Qc[2], Qc[3], Qn[1], frag_addr<1, KX>(xa, src), frag_addr<2, KX>(xb, srcb),
-            frag_addr<3, KX>(xb, srcb));
-  block8<9>(acc[0][4], acc[1][4], acc[2][4], acc[3][4], acc[0][5], acc[1][5], acc[2][5], acc[3][5], P[4], P[5],
-            Qc[0], Qc[1], Qc[2], Qc[3], Qn[2], frag_addr<2, KX>(xa, src), frag_addr<4, KX>(xb, srcb),
-            frag_addr<5, KX>(xb, srcb));
-  block8<9>(acc[0][6], acc[1][6], acc[2][6], acc[3][6], acc[0][7], acc[1][7], acc[2][7], acc[3][7], P[6], P[7],
-            Qc[0], Qc[1], Qc[2], Qc[3], Qn[3], frag_addr<3, KX>(xa, src), frag_addr<6, KX>(xb, srcb),
-            frag_addr<7, KX>(xb, srcb));
-}
-
-// ---- weights read as they lie ([K, N] row-major, N contiguous): the backward
-// dX products (dh = d_out * w2, dx = [da | db] * [w1; w3]) take their B
-// operand from the nn.Linear weights without a transposed copy.
-// B stage: 64 k rows of 512 bytes (256 n values), copied as they lie; the
-// 32-byte windows of a k row are XOR-swizzled by wsw(k row), and fragments
-// are read with ds_read_b64_tr_b16, which returns to lane (h = l / 16,
-// i = l % 16) column i of the 4 x 4 block of 16-bit values that the
-// group's source lanes 4 j + q address (row j, 4 values at column 4 q); two
-// such reads, 4 k rows apart, give a lane 8 consecutive k of one n.  A
-// 64-bit read cannot name half of an inline-assembly operand, so in this
-// variant all LDS reads are compiler loads (the compiler places the waits
-// for them) and only the MFMA groups are inline assembly.
+// ---- operands read as they lie ([K, N] row-major, N contiguous): the weights
+// of the backward dX products (dh = d_out * w2, dx = [da | db] * [w1; w3]) and
+// both operands of the weight gradients, without a transposed copy.
+// A unit is 64 k rows of 256 bytes (128 columns), copied as they lie (32-byte
+// windows of a k row XOR-swizzled by wsw(k row)); fragments are read with
+// ds_read_b64_tr_b16, which returns to lane (h = l / 16, i = l % 16) column i
+// of the 4 x 4 block of 16-bit values that the group's source lanes 4 j + q
+// address (row j, 4 values at column 4 q); two such reads, 4 k rows apart,
+// give a lane 8 consecutive k of one column.
 __device__ __forceinline__ int wsw(int r) { return (r & 3) | (((r >> 3) & 1) << 2); }
 
-// Lane's address of B fragment 0 (K half 0) within a stage, relative to the
-// stage base: k row 8 h + jq (+4 for the second read), window (8 wn + fr) for
-// the wave's 128 columns, fr = wsw(8 h + jq).  Fragment f: ^ (f << 5); the
-// second 32-deep half of the stage: + 32 rows.
-__device__ __forceinline__ uint32_t trb_base(int wn, int lane) {
+// Lane's address of fragment 0 (k 0..31) of a unit copied as it lies, relative
+// to the unit: k row 8 h + jq (+4 for the second read), the wave's first
+// window win0 (a multiple of the fragments it reads there), swizzled by
+// wsw(8 h + jq).  Fragment f: ^ (f << 5); the second 32 k rows: + TR_KHALF.
+__device__ __forceinline__ uint32_t tr_base(int win0, int lane) {
   const int h = lane >> 4, jq = (lane >> 2) & 3, q = lane & 3;
   const int fr = jq | ((h & 1) << 2);
-  return static_cast<uint32_t>(A_BYTES + (8 * h + jq) * 512 + ((8 * wn + fr) << 5) + 8 * q);
+  return static_cast<uint32_t>((8 * h + jq) * UNIT_ROW + ((win0 ^ fr) << 5) + 8 * q);
 }
-constexpr uint32_t TRB_KHALF = 32 * 512;
+constexpr uint32_t TR_KHALF = 32 * UNIT_ROW;
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
-// One B fragment: 8 consecutive k of the lane's n (two transposing reads).
-__device__ __forceinline__ bf16x8 trb_frag(uint32_t addr) {
+// One fragment of a unit copied as it lies: 8 consecutive k of the lane's
+// column (two transposing reads).
+__device__ __forceinline__ bf16x8 tr_frag(uint32_t addr) {
   typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
   const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(uintptr_t)addr);
-  const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(uintptr_t)(addr + 2048u));
+  const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(uintptr_t)(addr + 4u * UNIT_ROW));
   return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
-#define FMOE_MFA(c, a, b) "v_mfma_f32_16x16x32_bf16 " c ", " a ", " b ", " c "\n"
-// Four MFMAs of one B fragment: acc[0..3][j] += P[j] (x) Q[0..3].  The LDS
-// reads of this variant are compiler loads, so the compiler places exact
-// waits for them before the statement that consumes them.
-__device__ __forceinline__ void block4m(f32x4& c0, f32x4& c1, f32x4& c2, f32x4& c3, const bf16x8& p,
-                                        const bf16x8& q0, const bf16x8& q1, const bf16x8& q2, const bf16x8& q3) {
-  asm volatile(FMOE_MFA("%[c0]", "%[p]", "%[q0]") FMOE_MFA("%[c1]", "%[p]", "%[q1]")
-               FMOE_MFA("%[c2]", "%[p]", "%[q2]") FMOE_MFA("%[c3]", "%[p]", "%[q3]")
-               : [c0] "+v"(c0), [c1] "+v"(c1), [c2] "+v"(c2), [c3] "+v"(c3)
-               : [p] "v"(p), [q0] "v"(q0), [q1] "v"(q1), [q2] "v"(q2), [q3] "v"(q3)
+// ---- the K step -------------------------------------------------------------
+// Fragments of one half of an operand's stage: [k half][block].
+typedef bf16x8 AFrag[2][FM / 2];
+typedef bf16x8 BFrag[2][FN / 2];
+
+#define FMOE_MF(c, a, b) "v_mfma_f32_16x16x32_bf16 " c ", " a ", " b ", " c "\n"
+// Four MFMAs: two column blocks (p) x two row blocks (q).  The statement is
+// ordered against the fragment reads and the copies around it (memory
+// clobber), which fixes the interleaving; the fragment reads are compiler
+// loads, so the compiler waits for exactly those that a statement consumes.
+__device__ __forceinline__ void mfma4(f32x4& c00, f32x4& c10, f32x4& c01, f32x4& c11, const bf16x8& p0,
+                                      const bf16x8& p1, const bf16x8& q0, const bf16x8& q1) {
+  asm volatile(FMOE_MF("%[c00]", "%[p0]", "%[q0]") FMOE_MF("%[c10]", "%[p0]", "%[q1]")
+               FMOE_MF("%[c01]", "%[p1]", "%[q0]") FMOE_MF("%[c11]", "%[p1]", "%[q1]")
+               : [c00] "+v"(c00), [c10] "+v"(c10), [c01] "+v"(c01), [c11] "+v"(c11)
+               : [p0] "v"(p0), [p1] "v"(p1), [q0] "v"(q0), [q1] "v"(q1)
                : "memory");
 }
-#undef FMOE_MFA
+#undef FMOE_MF
 
-// kstep with B read as it lies.  Block x: MFMAs with P[2x], then the next
-// step's Q'[x] (A side, double buffered) and P[2x] (in place), MFMAs with
-// P[2x+1], then P[2x+1].  KH: the next fragments come from the second (1) or
-// first (0) 32-deep half of the stage at src.  (Measured against the
-// transposed-copy path on MI355X, outputs bit-identical: the two dX products
-// 1 % slower at C2 and 2 % at C5, less than the transposed copies cost.)
-template <int KH>
-__device__ __forceinline__ void kstep_t(f32x4 (&acc)[FM][FN], bf16x8 (&P)[FN], bf16x8 (&Qc)[4], bf16x8 (&Qn)[4],
-                                        uint32_t xa, uint32_t xbt, uint32_t src) {
-  constexpr int KX = KH ? 64 : 0;
-  const uint32_t bb = src + (KH ? TRB_KHALF : 0u);
-  typedef __attribute__((address_space(3))) bf16x8 lds_bf16x8;
-#define FMOE_BLK(X)                                                                                              \
-  block4m(acc[0][2 * X], acc[1][2 * X], acc[2][2 * X], acc[3][2 * X], P[2 * X], Qc[0], Qc[1], Qc[2], Qc[3]);        \
-  Qn[X] = *(const lds_bf16x8*)(uintptr_t)frag_addr<X, KX>(xa, src);                                                \
-  P[2 * X] = trb_frag(bb + (xbt ^ ((2u * X) << 5)));                                                              \
-  block4m(acc[0][2 * X + 1], acc[1][2 * X + 1], acc[2][2 * X + 1], acc[3][2 * X + 1], P[2 * X + 1], Qc[0], Qc[1],  \
-          Qc[2], Qc[3]);                                                                                          \
-  P[2 * X + 1] = trb_frag(bb + (xbt ^ ((2u * X + 1) << 5)));
-  FMOE_BLK(0)
-  FMOE_BLK(1)
-  FMOE_BLK(2)
-  FMOE_BLK(3)
-#undef FMOE_BLK
+// Quarter (I, J) of the wave's block, 64 deep: rows 32 I .. +31, columns
+// 64 J .. +63; every accumulator adds k 0..31 of the stage, then k 32..63.
+template <int I, int J>
+__device__ __forceinline__ void quarter(f32x4 (&acc)[FM][FN], const AFrag& a, const BFrag& b) {
+  __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+  for (int x = 0; x < 4; ++x) {
+    const int kh = x >> 1, n = (x & 1) * 2;
+    mfma4(acc[2 * I][4 * J + n], acc[2 * I + 1][4 * J + n], acc[2 * I][4 * J + n + 1], acc[2 * I + 1][4 * J + n + 1],
+          b[kh][n], b[kh][n + 1], a[kh][0], a[kh][1]);
+  }
+  __builtin_amdgcn_s_setprio(0);
+  barrier();
 }
 
 }  // namespace core
