@@ -1094,6 +1094,14 @@ struct WgradArgs {
   void* out_hi[FMOE_MAX_EXPERTS + 1];
 };
 
+// K chunks of a group of M rows: kc rows each, to the nearest count, so that
+// they can be made equally long (a multiple of 64 rows; the last may be
+// shorter or empty) and a group somewhat larger than kc stays whole.
+__host__ __device__ __forceinline__ int wgrad_chunks(int64_t M, int kc) {
+  const int n = static_cast<int>((M + kc / 2) / kc);
+  return n < 1 ? 1 : n;
+}
+
 __device__ __forceinline__ void group_rows(const WgradArgs& a, int g, int& row_base, int& M) {
   if (g < a.E) {
     row_base = a.offsets[g];
@@ -1133,29 +1141,37 @@ __global__ __launch_bounds__(core::NT, 1) void wgrad_tr_kernel(const WgradArgs a
   const uint32_t sbase = lds_addr(smem);
   const int tiles_m = (args.m_out + BM - 1) / BM, tiles_n = (args.n_out + BN - 1) / BN;
   const int tiles = tiles_m * tiles_n;
-  const int G = args.E + (args.rows_shared > 0 ? 1 : 0);
 
-  // ---- work unit -> (group, K chunk, output tile).  Units are dispatched in
-  // order (largest groups' chunks first when they come first); the hardware
-  // hands the next unit to the next free CU, which balances the uneven units.
-  int unit = blockIdx.x;
-  int g = 0, row_base = 0, M = 0, chunks = 0, pbase = 0;
-  for (; g < G; ++g) {
-    if (g < args.E) {
-      const int2 o = core::sload2(offsets + g);
-      row_base = o.x;
-      M = o.y - o.x;
-    } else {
+  // ---- work unit -> (group, K chunk, output tile): the shared group's chunks
+  // first (it is the largest group unless the routing is very skewed: at C5,
+  // 512 steps against 48, its units dispatched last left 168 CUs idle for
+  // 600 us), then the experts'.  The hardware hands the next unit to the next
+  // free CU, which balances the uneven units.  Lane e < E holds expert e's
+  // rows and first unit, as the tile map of the row products.
+  int g, row_base, M, chunks, pbase, unit = blockIdx.x;
+  {
+    const int s_chunks = args.rows_shared > 0 ? wgrad_chunks(args.rows_shared, args.kc) : 0;
+    if (unit < s_chunks * tiles) {
+      g = args.E;
       row_base = args.rows_routed;
       M = args.rows_shared;
+      chunks = s_chunks;
+      pbase = 0;
+    } else {
+      unit -= s_chunks * tiles;
+      const int lo = offsets[min(lane, args.E)], rows = offsets[min(lane + 1, args.E)] - lo;
+      const int nc = lane < args.E ? wgrad_chunks(rows, args.kc) : 0;
+      const int npart = nc > 1 ? nc : 0;
+      const int u_incl = wave_incl_scan(nc * tiles, lane), p_incl = wave_incl_scan(npart, lane);
+      if (unit >= __builtin_amdgcn_readlane(u_incl, 63)) return;
+      g = __builtin_ctzll(__ballot(u_incl > unit));
+      row_base = __builtin_amdgcn_readlane(lo, g);
+      M = __builtin_amdgcn_readlane(rows, g);
+      chunks = __builtin_amdgcn_readlane(nc, g);
+      pbase = (s_chunks > 1 ? s_chunks : 0) + __builtin_amdgcn_readlane(p_incl - npart, g);
+      unit -= __builtin_amdgcn_readlane(u_incl - nc * tiles, g);
     }
-    chunks = (M + args.kc - 1) / args.kc;
-    const int nu = chunks * tiles;
-    if (unit < nu) break;
-    unit -= nu;
-    if (chunks > 1) pbase += chunks;
   }
-  if (g >= G) return;
   const int chunk = unit / tiles, tile = unit - chunk * tiles;
   int tm = tile / tiles_n, tn = tile - tm * tiles_n;
   if (tiles % 8 == 0) {
@@ -1173,8 +1189,10 @@ __global__ __launch_bounds__(core::NT, 1) void wgrad_tr_kernel(const WgradArgs a
     }
   }
   const int m0 = tm * BM, n0 = tn * BN;
-  const int k_begin = chunk * args.kc;
-  const int k_end = min(M, k_begin + args.kc);
+  const int len = ((M + chunks - 1) / chunks + BK - 1) / BK * BK;  // rows of a chunk
+  const int k_begin = chunk * len;
+  const int k_end = min(M, k_begin + len);
+  // <= 0: no rows (a group without rows, whose gradient is zero, or an empty last chunk)
   const int nk = (k_end - k_begin + BK - 1) / BK;
   const bool shared_sep = (g >= args.E);
   const uint16_t* A = (shared_sep && args.a_shared) ? args.a_shared : args.a_routed + static_cast<int64_t>(row_base) * args.lda;
@@ -1287,71 +1305,72 @@ __global__ __launch_bounds__(core::NT, 1) void wgrad_tr_kernel(const WgradArgs a
     for (int n = 0; n < 4; ++n) read_b(b0, src, 0, n);
   };
 
-  if (gathered) form_gathered(0);
-  issue_a(0, 0);
-  issue_b(0, 0);
-  issue_b(0, 1);
-  issue_a(0, 1);
-  if (gathered) form_gathered(min(1, nk - 1));
-  issue_a(1, 0);
-  issue_b(1, 0);
-  issue_b(1, 1);
-  wait_copies(std::integral_constant<int, 5 * LU>{});
-  zero_tail(0, 0);
-  wait_lds_barrier();
-
   f32x4 acc[FM][FN];
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   asm volatile("s_nop 1" ::: "memory");  // VALU writes -> MFMA reads of the accumulators
-  read_first(sbase);
-  const bool late = w >= 4;
-  if (late) barrier();
+  if (nk > 0) {
+    if (gathered) form_gathered(0);
+    issue_a(0, 0);
+    issue_b(0, 0);
+    issue_b(0, 1);
+    issue_a(0, 1);
+    if (gathered) form_gathered(min(1, nk - 1));
+    issue_a(1, 0);
+    issue_b(1, 0);
+    issue_b(1, 1);
+    wait_copies(std::integral_constant<int, 5 * LU>{});
+    zero_tail(0, 0);
+    wait_lds_barrier();
+    read_first(sbase);
+    const bool late = w >= 4;
+    if (late) barrier();
 
-  for (int kt = 0; kt < nk; ++kt) {
-    asm volatile("" : "+v"(xa), "+v"(xb));
-    const uint32_t cur = sbase + (kt & 1) * STAGE, nxt = sbase + ((kt + 1) & 1) * STAGE;
-    // (0, 0)
+    for (int kt = 0; kt < nk; ++kt) {
+      asm volatile("" : "+v"(xa), "+v"(xb));
+      const uint32_t cur = sbase + (kt & 1) * STAGE, nxt = sbase + ((kt + 1) & 1) * STAGE;
+      // (0, 0)
 #pragma unroll
-    for (int n = 0; n < 4; ++n) read_b(b0, cur, 1, n);
-    issue_a(kt + 1, 1);
-    wait_copies(std::integral_constant<int, 5 * LU>{});  // B1 of this stage
-    wait_lds_barrier();
-    quarter<0, 0>(acc, a0, b0);
-    // (0, 1)
+      for (int n = 0; n < 4; ++n) read_b(b0, cur, 1, n);
+      issue_a(kt + 1, 1);
+      wait_copies(std::integral_constant<int, 5 * LU>{});  // B1 of this stage
+      wait_lds_barrier();
+      quarter<0, 0>(acc, a0, b0);
+      // (0, 1)
 #pragma unroll
-    for (int kh = 0; kh < 2; ++kh)
+      for (int kh = 0; kh < 2; ++kh)
 #pragma unroll
-      for (int n = 0; n < 4; ++n) read_b(b1, cur + UNIT, kh, n);
-    issue_a(kt + 2, 0);
-    wait_copies(std::integral_constant<int, 5 * LU>{});  // A1 of this stage
-    zero_tail(kt, 1);
-    wait_lds_barrier();
-    quarter<0, 1>(acc, a0, b1);
-    // (1, 0)
+        for (int n = 0; n < 4; ++n) read_b(b1, cur + UNIT, kh, n);
+      issue_a(kt + 2, 0);
+      wait_copies(std::integral_constant<int, 5 * LU>{});  // A1 of this stage
+      zero_tail(kt, 1);
+      wait_lds_barrier();
+      quarter<0, 1>(acc, a0, b1);
+      // (1, 0)
 #pragma unroll
-    for (int kh = 0; kh < 2; ++kh)
+      for (int kh = 0; kh < 2; ++kh)
 #pragma unroll
-      for (int m = 0; m < 2; ++m) read_a(a1, cur + UNIT, kh, m);
-    // gathered B: the offsets of stage kt + 2, whose ring slot landed a step ago
-    if (gathered) form_gathered(min(kt + 2, nk - 1));
-    issue_b(kt + 2, 0);
-    wait_copies(std::integral_constant<int, 4 * LU>{});  // A0, B0 of the next stage
-    zero_tail(kt + 1, 0);
-    wait_lds_barrier();
-    quarter<1, 0>(acc, a1, b0);
-    // (1, 1)
-    read_first(nxt);  // past the last stage: a harmless read
-    issue_b(kt + 2, 1);
-    wait_lds_barrier();
-    quarter<1, 1>(acc, a1, b1);
+        for (int m = 0; m < 2; ++m) read_a(a1, cur + UNIT, kh, m);
+      // gathered B: the offsets of stage kt + 2, whose ring slot landed a step ago
+      if (gathered) form_gathered(min(kt + 2, nk - 1));
+      issue_b(kt + 2, 0);
+      wait_copies(std::integral_constant<int, 4 * LU>{});  // A0, B0 of the next stage
+      zero_tail(kt + 1, 0);
+      wait_lds_barrier();
+      quarter<1, 0>(acc, a1, b0);
+      // (1, 1)
+      read_first(nxt);  // past the last stage: a harmless read
+      issue_b(kt + 2, 1);
+      wait_lds_barrier();
+      quarter<1, 1>(acc, a1, b1);
+    }
+    if (!late) barrier();
+    asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3\n" ::: "memory");  // MFMA results -> VALU reads
+    // the copies past the end have landed before the workgroup's LDS is given back
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
-  if (!late) barrier();
-  asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3\n" ::: "memory");  // MFMA results -> VALU reads
-  // the copies past the end have landed before the workgroup's LDS is given back
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
   // ---- epilogue: lane holds C[m0 + 128 (i / 2) + 32 wm + 16 (i % 2) + l % 16]
   //                           [n0 + 128 (j / 4) + 64 wn + 16 (j % 4) + 4 (l / 16) + 0..3]
@@ -1388,8 +1407,7 @@ __global__ __launch_bounds__(core::NT, 1) void wgrad_tr_kernel(const WgradArgs a
 // 64), written with 16-byte stores.  The loads of kWgradReduceBatch chunks are
 // issued together (a loop that waited for each chunk's loads before the next
 // paid one memory latency per chunk); the sums still run in chunk order,
-// from 0.  A group without rows gets a zero gradient (no work unit of the
-// product kernel writes it).
+// from 0.
 constexpr int kWgradReduceBatch = 8;
 
 __device__ __forceinline__ void store_grad8(const WgradArgs& a, int g, int64_t i0, const float (&v)[8]) {
@@ -1410,18 +1428,23 @@ __global__ __launch_bounds__(256) void wgrad_reduce_kernel(const WgradArgs args)
   const int g = blockIdx.y;
   int row_base, M;
   group_rows(args, g, row_base, M);
-  const int chunks = (M + args.kc - 1) / args.kc;
+  const int chunks = wgrad_chunks(M, args.kc);
   const int64_t mn = static_cast<int64_t>(args.m_out) * args.n_out;
   const int64_t i0 = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) * 8;
-  if (i0 >= mn || chunks == 1) return;
+  if (i0 >= mn || chunks <= 1) return;
   float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  if (chunks > 1) {
+  {
+    // first partial: the shared group's come first, then the experts'
     int pbase = 0;
-    for (int q = 0; q < g; ++q) {
-      int rb, Mq;
-      group_rows(args, q, rb, Mq);
-      const int cq = (Mq + args.kc - 1) / args.kc;
-      if (cq > 1) pbase += cq;
+    if (g < args.E) {
+      const int sc = wgrad_chunks(args.rows_shared, args.kc);
+      if (sc > 1) pbase = sc;
+      for (int q = 0; q < g; ++q) {
+        int rb, Mq;
+        group_rows(args, q, rb, Mq);
+        const int cq = wgrad_chunks(Mq, args.kc);
+        if (cq > 1) pbase += cq;
+      }
     }
     const float* src0 = args.partial + static_cast<int64_t>(pbase) * mn + i0;
     for (int c0 = 0; c0 < chunks; c0 += kWgradReduceBatch) {
@@ -1722,16 +1745,20 @@ extern "C" int fmoe_gateup_bwd_dx(const void* d_ab, const int32_t* offsets, int 
 }
 
 namespace fmoe {
-// Rows per K chunk of the weight gradient.  A work unit is (group, chunk,
-// output tile); the chunk is sized so that the largest unit is about half of
-// one CU's average share (tiles * rows / 64 K-steps over 256 CUs), which keeps
-// the skewed groups (one or two experts holding most rows) from leaving a long
-// tail.  A multiple of 64, at least 256 rows.
+// Rows per K chunk of the weight gradient (wgrad_chunks rounds a group to the
+// nearest count).  A work unit is (group, chunk, output tile); the chunk is
+// two thirds of one CU's average share (tiles * rows / 64 K steps over 256
+// CUs), so that skewed groups do not leave a long tail, and at least 768 rows:
+// a split tile costs 256 KB of fp32 partial per chunk, written and read once,
+// about six K steps' time.  Measured (dW2 + dW1|dW3, MI355X): T = 1021, d =
+// 768, 8 experts 136 -> 81 us, T = 4100 215 -> 185, T = 8192 332 -> 296, C2
+// 500 -> 482 us (one third of the share, rounded up: the left figures; the
+// whole share 532 us at C2, 172 at T = 4100).
 int64_t wgrad_kc(int64_t rows_routed, int64_t rows_shared, int64_t m_out, int64_t n_out) {
   const int64_t rows = rows_routed + rows_shared;
   const int64_t tiles = ceil_div(m_out, 256) * ceil_div(n_out, 256);
-  int64_t kc = (tiles * rows / 512) / 64 * 64;
-  return kc < 256 ? 256 : kc;
+  const int64_t kc = (tiles * rows / 384) / 64 * 64;
+  return kc < 768 ? 768 : kc;
 }
 }  // namespace fmoe
 
@@ -1739,7 +1766,7 @@ extern "C" size_t fmoe_weight_grad_workspace_bytes(int64_t rows_routed, int64_t 
                                                    int n_experts, int64_t m_out, int64_t n_out) {
   if (rows_routed < 0 || rows_shared < 0 || n_experts <= 0 || m_out <= 0 || n_out <= 0) return 0;
   const int64_t kc = wgrad_kc(rows_routed, rows_shared, m_out, n_out);
-  // sum over groups of ceil(M_g / kc) <= floor(rows / kc) + groups
+  // sum over groups of wgrad_chunks(M_g, kc) <= floor(rows / kc) + groups
   const int64_t chunks = (rows_routed + rows_shared) / kc + n_experts + 1;
   return static_cast<size_t>(chunks * m_out * n_out) * sizeof(float);
 }
@@ -1800,12 +1827,15 @@ extern "C" int fmoe_weight_grad(const void* a_routed, const void* a_shared, int6
     a.out_hi[g] = (m_split < m_out) ? out_hi[g] : nullptr;
   }
   const int64_t tiles = ceil_div(m_out, core::BM) * ceil_div(n_out, core::BN);
+  // sum over groups of wgrad_chunks(M_g) <= floor(rows / kc) + groups
   const int64_t max_chunks = (rows_routed + rows_shared) / a.kc + G;
   hipStream_t s = as_stream(stream);
   if (b_gather)
     wgrad_tr_kernel<true><<<dim3(max_chunks * tiles), dim3(core::NT), 0, s>>>(a, offsets);
   else
     wgrad_tr_kernel<false><<<dim3(max_chunks * tiles), dim3(core::NT), 0, s>>>(a, offsets);
+  // (no group can have two chunks: nothing to reduce)
+  if (wgrad_chunks(rows_routed, a.kc) == 1 && wgrad_chunks(rows_shared, a.kc) == 1) return launch_status();
   const int64_t mn = m_out * n_out;
   wgrad_reduce_kernel<<<dim3(ceil_div(mn, 256 * 8), G), dim3(256), 0, s>>>(a);
   return launch_status();
