@@ -133,24 +133,26 @@ __device__ __forceinline__ Tile locate_tile(const GemmArgs& a, const TileMap& m,
 
 // K-split of the last, partial round of tiles.  With T tiles on P
 // workgroups, the T mod P tiles of the last round would run on a fraction of
-// the CUs; instead each is split into S K ranges (S <= 4, R * S <= P, at
-// least 4 K steps per range) whose fp32 partials a split reduction adds in
+// the CUs; instead each is split into S K ranges (S <= 8, R * S <= P, at
+// least 8 K steps per range) whose fp32 partials a split reduction adds in
 // range order before the product's epilogue.  Work items: tiles 0 .. full-1
-// whole, then R * S ranges.
-// Only for runs of fewer than kSplitMaxRounds full rounds.  Measured on
-// MI355X (split minus whole, same process): at T=16384, d=768, I=2048 the
-// split gains 12 us on the down product (2 rounds, 32 K steps), 47 us on the
-// gate/up backward (2 rounds, 64 K steps) and 3 us on the down backward (6
-// rounds, 12 K steps) but loses 9 us on the gate/up forward (12 rounds, 12
-// K steps); at d=2048, I=1408, 64 experts (21 to 38 rounds) it loses 1 to
-// 15 us on every product.  Over many rounds the workgroups' finishing times
-// spread by about a tile anyway, and the partials' HBM traffic (written and
-// read once, 256 KB per range) is then not repaid.
+// whole, then R * S ranges.  A launch of fewer tiles than CUs takes every CU
+// for its ranges.  Measured on MI355X (d = 768, I = 2048, 8 experts; the grid
+// of such a launch was its tile count, which split nothing): gate/up dX at T
+// = 300 83 -> 40 us, T = 1021 84 -> 47, T = 2048 84 -> 59; dense T = 6100 84
+// -> 57.  Ranges of 4 steps (K = 768: three of 12) cost more in partials
+// (256 KB per range, written and read once) and in the reduction's launch
+// than they save: gate/up forward, dense T = 6100 64 -> 49 us without.
+// Only for runs of fewer than kSplitMaxRounds full rounds: over many rounds
+// the workgroups' finishing times spread by about a tile anyway (d = 2048, I =
+// 1408, 64 experts, 21 to 38 rounds: 1 to 15 us lost on every product).
 struct SplitPlan {
   int full, R, S;
   __device__ __forceinline__ int items() const { return full + R * S; }
 };
-constexpr int kSplitMaxS = 4;       // K ranges per split tile
+constexpr int kSplitMaxS = 8;       // K ranges per split tile
+constexpr int kSplitMinSteps = 8;   // K steps per range
+constexpr int kSplitBatch = 4;      // ranges whose partials a split reduction loads together
 constexpr int kSplitMaxRounds = 8;  // full rounds above which no tile is split
 constexpr int kReduceParts = 16;  // blocks of a split reduction per split tile, 16 rows each
 
@@ -160,8 +162,7 @@ __device__ __forceinline__ SplitPlan split_plan(const GemmArgs& a, int T, int P,
   if (a.split_ws == nullptr || T <= 0) return sp;
   const int R = T % P;
   if (R == 0 || T / P >= kSplitMaxRounds) return sp;
-  int S = min(P / R, kSplitMaxS);
-  S = min(S, nk / 4);
+  const int S = min(min(P / R, kSplitMaxS), nk / kSplitMinSteps);
   if (S < 2) return sp;
   sp.full = T - R;
   sp.R = R;
@@ -246,9 +247,11 @@ __device__ __forceinline__ void swiglu_bwd8(const uint4& dhv, const uint4& av, c
 // to bf16, through the wave's 4 KB of LDS one 16-row slice at a time, read
 // back as 16-byte row segments (64 registers, the accumulators are then
 // free); then the slices' a|b are loaded, computed and stored one after
-// another.  Row pointers are uniform (scalar registers); a lane adds one
-// offset.  Two slices of loads in flight spill 51 registers beside the main
-// loop's (C2 302 against 260 us, C5 1855 against 1510 us).
+// another, each slice's loads in registers of their own, so that the compiler
+// can issue them ahead (with the registers of the slice before: C2 310
+// against 253 us).  Two slices of loads issued up front spill 51 registers
+// beside the main loop's (C2 302 us, C5 1855 against 1500 us).  Row pointers
+// are uniform (scalar registers); a lane adds one offset.
 __device__ __forceinline__ void down_bwd_full_epilogue(const GemmArgs& args, const f32x4 (&acc)[core::FM][core::FN],
                                                        uint8_t* ep, int el, int64_t grow0, int col0) {
   using namespace core;
@@ -280,20 +283,24 @@ __device__ __forceinline__ void down_bwd_full_epilogue(const GemmArgs& args, con
   const uint32_t coff = static_cast<uint32_t>((el >> 4) * static_cast<int>(args.ldc0) + (el & 15) * 8) * 2u;
   const int64_t cstep = args.ldc0 * 2 * 4;
   const int64_t binter = args.inter * 2;  // bytes from a to b (and from da to db)
-  asm volatile("" ::: "memory");  // the loads are not hoisted into the staging above
-#pragma unroll
-  for (int i = 0; i < FM; ++i) {
-    uint4 pa[4], pb[4];
+  uint4 pa[FM][4], pb[FM][4];
+  auto load_slice = [&](int i) {
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       const uint8_t* rp = abase + (i * 4 + t) * astep;
-      pa[t] = load16(reinterpret_cast<const uint16_t*>(rp + aoff), true);
-      pb[t] = load16(reinterpret_cast<const uint16_t*>(rp + binter + aoff), true);
+      pa[i][t] = load16(reinterpret_cast<const uint16_t*>(rp + aoff), true);
+      pb[i][t] = load16(reinterpret_cast<const uint16_t*>(rp + binter + aoff), true);
     }
+  };
+  asm volatile("" ::: "memory");  // the loads are not hoisted into the staging above
+  load_slice(0);
+#pragma unroll
+  for (int i = 0; i < FM; ++i) {
+    if (i > 0) load_slice(i);
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       uint4 dav, dbv;
-      swiglu_bwd8(dhv[i][t], pa[t], pb[t], dav, dbv);
+      swiglu_bwd8(dhv[i][t], pa[i][t], pb[i][t], dav, dbv);
       uint8_t* rp = cbase + (i * 4 + t) * cstep;
       store16(reinterpret_cast<uint16_t*>(rp + coff), dav, true);
       store16(reinterpret_cast<uint16_t*>(rp + binter + coff), dbv, true);
@@ -731,25 +738,27 @@ __device__ __forceinline__ SplitTile split_tile(const float* ws, int P) {
   return t;
 }
 
-// Partial values o .. o + 7 of the S ranges, summed in range order from 0
-// (all kSplitMaxS loads issued first; ranges past S re-read range S - 1 and
-// are not added).
+// Partial values o .. o + 7 of the S ranges, summed in range order from 0 (the
+// loads of kSplitBatch ranges issued together; ranges past S re-read range
+// S - 1 and are not added).
 __device__ __forceinline__ void sum_ranges8(const SplitTile& t, int o, float* acc) {
   using namespace core;
-  float4 u[kSplitMaxS][2];
-#pragma unroll
-  for (int s = 0; s < kSplitMaxS; ++s) {
-    const float* p = t.src0 + static_cast<int64_t>(min(s, t.S - 1)) * BM * BN + o;
-    u[s][0] = *reinterpret_cast<const float4*>(p);
-    u[s][1] = *reinterpret_cast<const float4*>(p + 4);
-  }
 #pragma unroll
   for (int e = 0; e < 8; ++e) acc[e] = 0.0f;
+  for (int s0 = 0; s0 < t.S; s0 += kSplitBatch) {
+    float4 u[kSplitBatch][2];
 #pragma unroll
-  for (int s = 0; s < kSplitMaxS; ++s) {
-    const float v[8] = {u[s][0].x, u[s][0].y, u[s][0].z, u[s][0].w, u[s][1].x, u[s][1].y, u[s][1].z, u[s][1].w};
+    for (int s = 0; s < kSplitBatch; ++s) {
+      const float* p = t.src0 + static_cast<int64_t>(min(s0 + s, t.S - 1)) * BM * BN + o;
+      u[s][0] = *reinterpret_cast<const float4*>(p);
+      u[s][1] = *reinterpret_cast<const float4*>(p + 4);
+    }
 #pragma unroll
-    for (int e = 0; e < 8; ++e) acc[e] = (s < t.S) ? acc[e] + v[e] : acc[e];
+    for (int s = 0; s < kSplitBatch; ++s) {
+      const float v[8] = {u[s][0].x, u[s][0].y, u[s][0].z, u[s][0].w, u[s][1].x, u[s][1].y, u[s][1].z, u[s][1].w};
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[e] = (s0 + s < t.S) ? acc[e] + v[e] : acc[e];
+    }
   }
 }
 
@@ -1537,7 +1546,11 @@ int launch_rows(GemmArgs& a, int64_t rows_routed, int64_t rows_shared, int E, vo
   const int64_t tiles = (rows_routed / core::BM + E + ceil_div(rows_shared, core::BM)) * tiles_n;
   if (tiles <= 0) return FMOE_OK;
   if (!all_small) {
-    const int64_t grid = tiles < device_cus() ? tiles : device_cus();
+    // A launch of fewer tiles than CUs still takes every CU if its tiles can be
+    // split along K (ranges of kSplitMinSteps steps at least).
+    const int64_t cus = device_cus();
+    if (a.K / core::BK < 2 * kSplitMinSteps) a.split_ws = nullptr;
+    const int64_t grid = (a.split_ws == nullptr && tiles < cus) ? tiles : cus;
     // A run of kSplitMaxRounds full rounds or more never splits (split_plan);
     // sum over groups of ceil(M_g / BM) >= ceil(rows / BM) bounds the tile
     // count from below, so such a run skips the header and the reduction.
@@ -1550,15 +1563,15 @@ int launch_rows(GemmArgs& a, int64_t rows_routed, int64_t rows_shared, int E, vo
     }
     if (!gathered) rows_gemm_kernel<MODE, false><<<dim3(grid), dim3(core::NT), 0, as_stream(stream)>>>(a, a.offsets);
     if (a.split_ws != nullptr) {
+      // at most half of the CUs' tiles are split (R S <= grid, S >= 2)
+      const dim3 rgrid((tiles < cus / 2 ? tiles : cus / 2) * kReduceParts);
       if constexpr (MODE == DOWN_FWD || MODE == GATEUP_BWD)
-        split_reduce_kernel<<<dim3(grid * kReduceParts), dim3(256), 0, as_stream(stream)>>>(
-            a.split_ws, static_cast<int>(grid), a.c0, a.ldc0);
+        split_reduce_kernel<<<rgrid, dim3(256), 0, as_stream(stream)>>>(a.split_ws, static_cast<int>(grid), a.c0,
+                                                                       a.ldc0);
       else if constexpr (MODE == GATEUP_FWD)
-        split_reduce_gateup_kernel<<<dim3(grid * kReduceParts), dim3(256), 0, as_stream(stream)>>>(
-            a, static_cast<int>(grid));
+        split_reduce_gateup_kernel<<<rgrid, dim3(256), 0, as_stream(stream)>>>(a, static_cast<int>(grid));
       else
-        split_reduce_down_bwd_kernel<<<dim3(grid * kReduceParts), dim3(256), 0, as_stream(stream)>>>(
-            a, static_cast<int>(grid));
+        split_reduce_down_bwd_kernel<<<rgrid, dim3(256), 0, as_stream(stream)>>>(a, static_cast<int>(grid));
     }
   }
   if constexpr (kHasSmall) {
