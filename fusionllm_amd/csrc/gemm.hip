@@ -1502,9 +1502,18 @@ int check_row_product(int n_experts, int64_t rows_routed, int64_t rows_shared, i
 }
 
 // Row counts up to which a launch sends groups of <= kSmallM rows to the
-// small-group kernel (decode-sized batches); larger launches use the tiled
-// kernel for every group.
+// small-group kernel (decode-sized batches), if they have at most kSmallAvgRows
+// routed rows per expert, or no group can exceed 2 kSmallM rows; all other
+// launches use the tiled kernel for every group.  Both kernels cost their
+// share when groups of both kinds occur, and the tiled one is the faster from
+// about 8 rows per group: it reads a weight once per 256 rows, the small one
+// once per 16 to 128.  Measured (gate/up + down forward, MI355X, small kernel
+// for groups of <= 128 rows -> tiled kernel): 64 experts, d = 2048, I = 1408,
+// top-6: T = 200 367 -> 285 us, T = 340 452 -> 289, T = 580 592 -> 298 (T = 64, 6
+// rows per expert: 271 against 295 us); 8 experts, d = 768, I = 2048, top-2: T =
+// 150 82 -> 59, T = 300 104 -> 62; 16 experts, top-4: T = 400 161 -> 72.
 constexpr int64_t kSmallLaunchRows = 4096;
+constexpr int64_t kSmallAvgRows = 8;
 
 // Compute units of the current device (the persistent grid size), cached per
 // device ordinal.
@@ -1534,7 +1543,10 @@ int launch_rows(GemmArgs& a, int64_t rows_routed, int64_t rows_shared, int E, vo
   constexpr int TN_COLS = (MODE == GATEUP_FWD) ? core::BN / 2 : core::BN;
   const int64_t tiles_n = ceil_div(a.N, TN_COLS);
   constexpr bool kHasSmall = (MODE == GATEUP_FWD || MODE == DOWN_FWD);
-  a.small_max = (kHasSmall && rows_routed + rows_shared <= kSmallLaunchRows) ? kSmallM : 0;
+  a.small_max = (kHasSmall && rows_routed + rows_shared <= kSmallLaunchRows &&
+                 (rows_routed <= kSmallAvgRows * E || (rows_routed <= 2 * kSmallM && rows_shared <= kSmallM)))
+                    ? kSmallM
+                    : 0;
   // A routed group has at most rows_routed rows: when no group can exceed
   // 2 kSmallM rows (the small kernel takes a larger group as two slabs), the
   // tiled kernel (and its split reduction) would have nothing to do.  This
