@@ -185,7 +185,6 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_scatter_kernel(
   const int wave = threadIdx.x >> 6;
   for (int e = threadIdx.x; e < E; e += blockDim.x)
     running[e] = block_base[static_cast<int64_t>(blockIdx.x) * E + e];
-  const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   for (int round = 0; round < kSlotsPerThread; ++round) {
     for (int i = threadIdx.x; i < kDispWaves * E; i += blockDim.x) wcount[i / E][i % E] = 0;
     __syncthreads();
@@ -193,17 +192,7 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_scatter_kernel(
     const int e_raw = s < n_slots ? idx[s] : -1;
     const bool valid = static_cast<unsigned>(e_raw) < static_cast<unsigned>(E);
     const int e = valid ? e_raw : -1;
-    // Rank among lanes of this wave with the same expert (lower lanes first).
-    uint64_t pending = __ballot(valid);
-    int rank = 0;
-    while (pending) {
-      const int leader = __ffsll(static_cast<unsigned long long>(pending)) - 1;
-      const int le = __shfl(e, leader);
-      const uint64_t m = __ballot(e == le);
-      if (e == le) rank = __popcll(m & lt_mask);
-      if (lane == leader) wcount[wave][le] = __popcll(m);
-      pending &= ~m;
-    }
+    const int rank = rank_in_wave(e, valid, lane, wcount[wave]);
     __syncthreads();
     if (valid) {
       int pos = running[e] + rank;
@@ -255,17 +244,7 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_scatter_copy_kernel(
   __syncthreads();
   const bool valid = static_cast<unsigned>(e_raw) < static_cast<unsigned>(E);
   const int e = valid ? e_raw : -1;
-  const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  uint64_t pending = __ballot(valid);
-  int rank = 0;
-  while (pending) {
-    const int leader = __ffsll(static_cast<unsigned long long>(pending)) - 1;
-    const int le = __shfl(e, leader);
-    const uint64_t m = __ballot(e == le);
-    if (e == le) rank = __popcll(m & lt_mask);
-    if (lane == leader) wcount[wave][le] = __popcll(m);
-    pending &= ~m;
-  }
+  const int rank = rank_in_wave(e, valid, lane, wcount[wave]);
   __syncthreads();
   int pos = -1;
   if (valid) {
@@ -331,17 +310,7 @@ __global__ __launch_bounds__(kDispThreads) void dispatch_small_kernel(
   const int e_raw = s < n_slots ? idx[s] : -1;
   const bool valid = static_cast<unsigned>(e_raw) < static_cast<unsigned>(E);
   const int e = valid ? e_raw : -1;
-  const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  uint64_t pending = __ballot(valid);
-  int rank = 0;
-  while (pending) {
-    const int leader = __ffsll(static_cast<unsigned long long>(pending)) - 1;
-    const int le = __shfl(e, leader);
-    const uint64_t m = __ballot(e == le);
-    if (e == le) rank = __popcll(m & lt_mask);
-    if (lane == leader) wcount[wave][le] = __popcll(m);
-    pending &= ~m;
-  }
+  const int rank = rank_in_wave(e, valid, lane, wcount[wave]);
   __syncthreads();
   scan_wave_counts<kDispWaves>(wcount, E, start);
   __syncthreads();

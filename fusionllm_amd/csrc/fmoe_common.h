@@ -74,6 +74,25 @@ __device__ __forceinline__ int wave_incl_scan(int v, int lane) {
   return v;
 }
 
+// Rank of this lane's slot among the wave's earlier lanes with the same expert
+// e (< 64), for valid lanes, and the wave's count per expert (wcount[e], set by
+// the expert's first lane; experts without slots are not touched).  The lanes
+// of one expert are found by one ballot per bit of e: the same six steps for
+// any spread of experts.  (A round per distinct expert, each a cross-lane read
+// and a ballot: dispatch of 96 slots over 64 experts 9.9 against 6.2 us.)
+__device__ __forceinline__ int rank_in_wave(int e, bool valid, int lane, int* wcount) {
+  uint64_t same = __ballot(valid);
+#pragma unroll
+  for (int b = 0; b < 6; ++b) {
+    const bool bit = (e >> b) & 1;
+    const uint64_t on = __ballot(bit);
+    same &= bit ? on : ~on;
+  }
+  const int rank = __popcll(same & ((uint64_t(1) << lane) - 1));
+  if (valid && rank == 0) wcount[e] = __popcll(same);
+  return rank;
+}
+
 // Expert offsets of a counting sort from per-wave counts (E <= 64):
 // start[q] = sum over experts q' < q of sum_w wcount[w][q'], start[E] = the
 // total.  Wave 0 does it: lane q adds its expert's W wave counts (independent
