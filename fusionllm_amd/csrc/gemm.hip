@@ -572,14 +572,18 @@ __global__ __launch_bounds__(core::NT, 1) void rows_gemm_kernel(const GemmArgs a
     int el = lane;
     asm volatile("" : "+v"(el));
     if (e_slot >= 0) {
-      // K-split range: fp32 partial of the 256 x 256 tile (local row-major)
+      // K-split range: fp32 partial of the 256 x 256 tile (local row-major),
+      // 16-row slices without valid rows left out (the reduction reads none)
       float* part = args.split_ws + static_cast<int64_t>(e_slot) * BM * BN;
+      const Tile t = locate_tile(args, map, tiles_n, e_tile);
+      const int rows_valid = t.M - t.tm * BM;
 #pragma unroll
       for (int i = 0; i < FM; ++i)
+        if (wm * WTM + i * 16 < rows_valid)
 #pragma unroll
-        for (int j = 0; j < FN; ++j)
-          *reinterpret_cast<f32x4*>(part + (wm * WTM + i * 16 + (el & 15)) * BN + wn * WTN + j * 16 + (el >> 4) * 4) =
-              acc[i][j];
+          for (int j = 0; j < FN; ++j)
+            *reinterpret_cast<f32x4*>(part + (wm * WTM + i * 16 + (el & 15)) * BN + wn * WTN + j * 16 + (el >> 4) * 4) =
+                acc[i][j];
     } else {
       const Tile t = locate_tile(args, map, tiles_n, e_tile);
       const int rows_valid = min(t.M - t.tm * BM, BM);
@@ -731,9 +735,9 @@ __device__ __forceinline__ SplitTile split_tile(const float* ws, int P) {
   const int4 h0 = hdr[0];
   const int r = blockIdx.x / kReduceParts;
   SplitTile t;
-  t.active = r < h0.x;
   t.S = h0.y;
-  t.d = t.active ? hdr[1 + r] : make_int4(0, 0, 0, 0);
+  t.d = r < h0.x ? hdr[1 + r] : make_int4(0, 0, 0, 0);
+  t.active = static_cast<int>(blockIdx.x % kReduceParts) * 16 < t.d.y;  // the block has valid rows
   t.src0 = ws + static_cast<int64_t>(r) * h0.y * BM * BN;
   return t;
 }
