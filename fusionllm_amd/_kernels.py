@@ -56,6 +56,32 @@ def _stream() -> ctypes.c_void_p:
     return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
 
 
+def stream_handle() -> int:
+    """The current device's current stream as an integer (for the native launch sequences)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+
+
+_BLOCK_HOST = None
+
+
+def block_host():
+    """The native forward and backward launch sequences (csrc/block_host.cpp), or None while
+    per-entry-point timing is on (the wrappers below record it).  Raises if the module has not
+    been built."""
+    global _BLOCK_HOST
+    if _TIMER is not None:
+        return None
+    if _BLOCK_HOST is None:
+        _lib.load()
+        try:
+            from . import _block_host
+        except ImportError as e:
+            raise FileNotFoundError("fusionllm_amd/_block_host.so is missing or does not load: build the extension "
+                                    "first (python -m fusionllm_amd.build or __graft_entry__.build())") from e
+        _BLOCK_HOST = _block_host
+    return _BLOCK_HOST
+
+
 def _req(t: torch.Tensor, name: str, dtype: torch.dtype | None = None) -> int:
     if not t.is_cuda:
         raise RuntimeError(f"{name} must be a ROCm device tensor (got {t.device})")

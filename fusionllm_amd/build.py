@@ -3,7 +3,8 @@
 Usage: python -m fusionllm_amd.build   (or fusionllm_amd.build.build_library())
 
 Every .hip file under csrc/ is compiled for gfx950 only and linked into one
-shared library next to this file.  Compiler flags:
+shared library next to this file; csrc/block_host.cpp becomes the Python
+module _block_host beside it.  Compiler flags of the kernels:
   -ffp-contract=off   every fused multiply-add in the kernels is explicit, so
                       the rounding steps are the written ones;
   -packed-fp32-ops off, per the MI355X pool's guidance (hipcc's host pass
@@ -21,6 +22,7 @@ PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR / "csrc"
 BUILD_DIR = PKG_DIR / "_build"
 LIB_PATH = PKG_DIR / "libfusionmoe.so"
+HOST_PATH = PKG_DIR / "_block_host.so"
 ARCH = "gfx950"
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -49,8 +51,33 @@ def _compile(src: Path) -> Path:
     return obj
 
 
+def build_host_module() -> Path:
+    """Compile csrc/block_host.cpp (the block's launch sequence on torch's C++ API,
+    linked against libfusionmoe.so next to it) into the module _block_host."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    tmp = HOST_PATH.with_suffix(".so.tmp")
+    includes = [*cpp_extension.include_paths(), sysconfig.get_path("include")]
+    libdir = cpp_extension.library_paths()[0]
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+           "-DTORCH_EXTENSION_NAME=_block_host",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *[f"-I{i}" for i in includes], str(CSRC / "block_host.cpp"), "-o", str(tmp),
+           f"-L{PKG_DIR}", "-lfusionmoe", f"-L{libdir}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10",
+           "-Wl,-rpath,$ORIGIN"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"{cmd[0]} failed on block_host.cpp:\n{res.stdout}\n{res.stderr}")
+    os.replace(tmp, HOST_PATH)
+    return HOST_PATH
+
+
 def build_library(verbose: bool = True) -> Path:
-    """Compile every kernel source and link libfusionmoe.so; returns its path."""
+    """Compile every kernel source, link libfusionmoe.so and build the host module on it;
+    returns the library's path."""
     BUILD_DIR.mkdir(exist_ok=True)
     sources = sorted(CSRC.glob("*.hip"))
     if not sources:
@@ -63,6 +90,7 @@ def build_library(verbose: bool = True) -> Path:
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stdout}\n{res.stderr}")
     os.replace(tmp, LIB_PATH)
+    build_host_module()
     if verbose:
         print(f"built {LIB_PATH} from {len(sources)} sources", file=sys.stderr)
     return LIB_PATH

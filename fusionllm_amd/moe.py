@@ -252,6 +252,14 @@ def _forward_pass(meta, x, gate_w, gate_b, weights, residual=None, counts_host=N
     w1s, w3s, w2s = wb[0::3][:G], wb[1::3][:G], wb[2::3][:G]
     gather = gathers_rows(T, k, has_shared)
 
+    if T > K.ROUTER_SMALL_T and d <= 2048 and not gather:
+        host = K.block_host()
+        if host is not None:
+            # the sequence below in one native call (same entry points, same order)
+            idx, idx64, w, v, counts, offsets, perm, pos, x_perm, ab, h, o, y = host.forward(
+                xb, gwb, gbb, w1s, w3s, w2s, k, inter, rs, has_shared, out_dtype, residual, counts_host,
+                K.stream_handle())
+            return xb, gwb, wb, idx, idx64, w, v, counts, offsets, perm, pos, x_perm, ab, h, o, y
     if 0 < T <= K.TINY_BATCH and T * E <= 64 and d <= 2048:
         # decode-sized: routing and dispatch in one launch (one workgroup)
         idx, idx64, w, v, counts, offsets, perm, pos, x_perm = K.route_dispatch(xb, gwb, gbb, k, rs)
@@ -332,6 +340,16 @@ def _backward_pass(ctx, saved, dy):
     rows_r, rows_s = T * k, (T if has_shared else 0)
     gw_dtype, gb_dtype, w_dtypes = ctx.param_dtypes
 
+    gather = x_perm is None or (x_perm.shape[0] == 0 and rows_r > 0)
+    host = None if gather else K.block_host()
+    if host is not None:
+        # the sequence below in one native call (same entry points, same order)
+        dx_rows, d_logits, dgw, dgb, *dws = host.backward(
+            dy, xb, gwb, w, v, offsets, perm, x_perm, ab, h, o, w1s, w3s, w2s, k, inter, rs, has_shared, gw_dtype,
+            w_dtypes[:3 * G], K.stream_handle())
+        return (dx_rows, d_logits, dgw, _gate_bias_grad(dgb, gb_dtype),
+                _expert_grads(ctx, dws[0::3], dws[1::3], dws[2::3], wb))
+
     # Combine backward: routed rows get dy*w (bf16), slots get <dy, o>.
     d_o, d_w = K.combine_bwd(dy, o, w, perm, k)
     dy_sh = _as_bf16(dy).contiguous() if has_shared else None
@@ -346,26 +364,32 @@ def _backward_pass(ctx, saved, dy):
     dx_rows = K.gateup_bwd_dx(d_ab, offsets, E, rows_r, rows_s, w1s, w3s, d)
     dw1 = [torch.empty(inter, d, dtype=w_dtypes[3 * g], device=xb.device) for g in range(G)]
     dw3 = [torch.empty(inter, d, dtype=w_dtypes[3 * g + 1], device=xb.device) for g in range(G)]
-    gather = x_perm is None or (x_perm.shape[0] == 0 and rows_r > 0)
     K.weight_grad(d_ab, None, xb if gather else x_perm, xb if has_shared else None, offsets, E, rows_r, rows_s,
                   inter, dw1, dw3, w_dtypes[0], b_gather=perm if gather else None, k=k, tag="w13")
     # Router: logits gradient, gate weight/bias gradient.
     d_logits, dgw, dgb = K.router_bwd(d_w, v, perm, offsets, xb, E, rs, gw_dtype)
-    if dgb.dtype != gb_dtype:
-        dgb = dgb.to(gb_dtype)
+    return dx_rows, d_logits, dgw, _gate_bias_grad(dgb, gb_dtype), _expert_grads(ctx, dw1, dw3, dw2, wb)
 
+
+def _gate_bias_grad(dgb, dtype):
+    return dgb if dgb.dtype == dtype else dgb.to(dtype)
+
+
+def _expert_grads(ctx, dw1, dw3, dw2, wb):
+    """Gradients in the order of the weights: None for experts that got no tokens (by the
+    forward's host copy of the counts).  Without that copy (the graph-capturable operator)
+    every expert gets its gradient: zeros for experts without rows."""
+    E = ctx.meta[0]
     grads_w = [None] * len(wb)
     counts = None
     if getattr(ctx, "counts_host", None) is not None:
         ctx.counts_event.synchronize()
         counts = ctx.counts_host.tolist()
-    # Without the host copy of the counts (the graph-capturable operator)
-    # every expert gets its gradient: zeros for experts without rows.
-    for g in range(G):
+    for g in range(len(dw1)):
         if counts is not None and g < E and counts[g] == 0:
             continue
         grads_w[3 * g], grads_w[3 * g + 1], grads_w[3 * g + 2] = dw1[g], dw3[g], dw2[g]
-    return dx_rows, d_logits, dgw, dgb, grads_w
+    return grads_w
 
 
 class _MoEBlockFunction(torch.autograd.Function):
