@@ -1,0 +1,135 @@
+"""The dispatch rules of the tiled products and the native launch sequence at
+the sizes where they change: K splits of small launches, the chunks of the
+weight gradients, the small-group limit, the top-k over a token's lanes."""
+import pytest
+import torch
+
+from fusionllm_amd import DeepSeekMoE, configs
+from fusionllm_amd import _kernels as K
+
+pytestmark = pytest.mark.gpu
+
+
+def _bf(*shape, g, scale=1.0):
+    return (torch.randn(*shape, generator=g) * scale).bfloat16()
+
+
+def _groups(counts, device):
+    off = torch.tensor([0, *torch.tensor(counts).cumsum(0).tolist()], dtype=torch.int32, device=device)
+    return off, sum(counts)
+
+
+# bf16 outputs of fp32 sums of bf16 operands: one rounding (2^-9 relative) and
+# the sums' own error (K 2^-24, below it); rel-L2 bound 4e-3 as for one
+# bf16 rounding of every element.
+BOUND = 4e-3
+
+
+def _rel(a, b):
+    return float((a.double() - b.double()).norm() / b.double().norm().clamp_min(1e-30))
+
+
+@pytest.mark.parametrize("counts,shared,d,I", [
+    ([0, 15, 16, 17], 0, 512, 1024),        # 16 steps: the fewest that split; slices of 16 rows
+    ([255, 256, 257, 1], 300, 1024, 576),   # tile edges, columns that do not fill a tile
+    ([700, 0, 3, 120], 1000, 64, 1088),     # one K step forward, two ranges of the down product
+    ([130] * 16, 0, 1024, 512),             # 8 to 16 rows per expert and more: the small-group limit
+])
+def test_row_products_of_small_launches(gpu_device, counts, shared, d, I):
+    D = gpu_device
+    g = torch.Generator().manual_seed(sum(counts) + d)
+    E, G = len(counts), len(counts) + (1 if shared else 0)
+    off, rr = _groups(counts, D)
+    x, h = _bf(rr, d, g=g).to(D), _bf(rr + shared, I, g=g).to(D)
+    xs = _bf(shared, d, g=g).to(D) if shared else None
+    dab = _bf(rr + shared, 2 * I, g=g, scale=0.1).to(D)
+    w1 = [_bf(I, d, g=g, scale=0.05).to(D) for _ in range(G)]
+    w3 = [_bf(I, d, g=g, scale=0.05).to(D) for _ in range(G)]
+    w2 = [_bf(d, I, g=g, scale=0.05).to(D) for _ in range(G)]
+    ab, _ = K.gateup_fwd(x, xs, off, E, w1, w3, I)
+    o = K.down_fwd(h, off, E, rr, shared, w2, d)
+    dx = K.gateup_bwd_dx(dab, off, E, rr, shared, w1, w3, d)
+    bounds = [0, *torch.tensor(counts).cumsum(0).tolist()] + ([rr + shared] if shared else [])
+    xa = torch.cat([x, xs]) if shared else x
+    for q in range(G):
+        r = slice(bounds[q], bounds[q + 1])
+        if r.stop == r.start:
+            continue
+        f = lambda t: t.float()
+        assert _rel(ab[r, :I], f(xa[r]) @ f(w1[q]).t()) < BOUND
+        assert _rel(ab[r, I:], f(xa[r]) @ f(w3[q]).t()) < BOUND
+        assert _rel(o[r], f(h[r]) @ f(w2[q]).t()) < BOUND
+        assert _rel(dx[r], f(dab[r, :I]) @ f(w1[q]) + f(dab[r, I:]) @ f(w3[q])) < BOUND
+
+
+@pytest.mark.parametrize("counts,shared,m,n", [
+    ([0, 1, 63, 64, 65], 0, 256, 320),       # groups without rows, one stage and its edges
+    ([1151, 1152, 1153, 0], 0, 512, 256),    # one chunk or two (kc = 768: from 1152 rows)
+    ([100, 2000], 5000, 64, 704),            # shared group in several chunks, a partial tile
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_weight_gradient_chunks(gpu_device, counts, shared, m, n, dtype):
+    D = gpu_device
+    g = torch.Generator().manual_seed(sum(counts) + m)
+    E, G = len(counts), len(counts) + (1 if shared else 0)
+    off, rr = _groups(counts, D)
+    a, b = _bf(rr, m, g=g).to(D), _bf(rr, n, g=g).to(D)
+    sa, sb = (_bf(shared, m, g=g).to(D), _bf(shared, n, g=g).to(D)) if shared else (None, None)
+    outs = [torch.full((m, n), float("nan"), dtype=dtype, device=D) for _ in range(G)]
+    K.weight_grad(a, sa, b, sb, off, E, rr, shared, m, outs, None, dtype)
+    bounds = [0, *torch.tensor(counts).cumsum(0).tolist()]
+    for q in range(G):
+        A, B = (sa, sb) if q == E else (a[bounds[q]:bounds[q + 1]], b[bounds[q]:bounds[q + 1]])
+        want = A.double().t() @ B.double()
+        if A.shape[0] == 0:
+            assert not outs[q].any()  # a group without rows: zeros
+        else:
+            # fp32: sums of at most 5000 exact products, error about sqrt(rows) 2^-24 per unit
+            assert _rel(outs[q], want) < (BOUND if dtype == torch.bfloat16 else 2e-6)
+
+
+@pytest.mark.parametrize("T,shared,autocast", [(129, 1, False), (300, 0, False), (700, 1, True)])
+def test_native_sequence_equals_the_entry_points(gpu_device, T, shared, autocast):
+    # With timing on, the block runs through the per-entry-point wrappers; the
+    # native sequence launches the same kernels: bit-equal.
+    cfg = configs.BlockConfig("native", T, dim=256, inter=512, n_experts=8, topk=2, n_shared=shared, bias="skew")
+    data = configs.make_block(cfg, seed=5)
+    res = []
+    for timer in ({}, None):
+        torch.manual_seed(0)
+        m = DeepSeekMoE(cfg.moe_config())
+        m.load_state_dict(data.state_dict())
+        m = m.to(gpu_device, torch.float32 if autocast else torch.bfloat16)
+        x = data.x.to(gpu_device, torch.float32 if autocast else torch.bfloat16).requires_grad_()
+        K.set_timer(timer)
+        try:
+            with torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast):
+                y = m(x)
+            y.backward(data.dy.to(gpu_device, y.dtype))
+        finally:
+            K.set_timer(None)
+        res.append([y.detach(), x.grad, m._last_indices, *[p.grad for _, p in m.named_parameters()]])
+    for a, b in zip(*res):
+        assert (a is None) == (b is None)
+        assert a is None or torch.equal(a, b)
+
+
+@pytest.mark.parametrize("E,k", [(1, 1), (15, 8), (16, 8), (17, 8), (33, 5), (64, 8)])
+def test_topk_ties_and_nan_across_lanes(gpu_device, E, k):
+    # Scores that tie across lanes and within one, and NaN scores: the lowest
+    # expert index wins, NaN first, as torch's stable descending sort orders.
+    T, d = 200, 64
+    g = torch.Generator().manual_seed(E)
+    x = torch.zeros(T, d).bfloat16()
+    x[:, 0] = 1.0
+    gw = torch.zeros(E, d).bfloat16()
+    gw[:, 0] = torch.randint(-2, 3, (E,), generator=g).bfloat16()
+    x[3, 1] = float("nan")  # a token whose every score is NaN
+    gb = torch.zeros(E).bfloat16()
+    idx, _, w, v = K.router_fwd(x.to(gpu_device), gw.to(gpu_device), gb.to(gpu_device), k, 1.0)
+    want = torch.sort(gw[:, 0].float(), descending=True, stable=True).indices[:k]
+    got = idx.cpu().long()
+    keep = torch.ones(T, dtype=torch.bool)
+    keep[3] = False
+    assert torch.equal(got[keep], want.expand(T - 1, k))
+    assert torch.equal(got[3], torch.arange(k)) and torch.isnan(v[3]).all()
