@@ -7,8 +7,9 @@ shared library next to this file; csrc/block_host.cpp becomes the Python
 module _block_host beside it.  Compiler flags of the kernels:
   -ffp-contract=off   every fused multiply-add in the kernels is explicit, so
                       the rounding steps are the written ones;
-  -packed-fp32-ops off, per the MI355X pool's guidance (hipcc's host pass
-                      warns that it does not know the feature; harmless).
+  -packed-fp32-ops off: some packed fp32 forms have given wrong results on
+                      this hardware (hipcc's host pass warns that it does not
+                      know the feature; harmless).
 """
 from __future__ import annotations
 

@@ -13,6 +13,8 @@
 // Reference: FusionLLM models/moe.py:79-87 (forward) and its autograd.
 #include <torch/extension.h>
 
+#include <algorithm>
+#include <stdexcept>
 #include <string>
 #include <vector>
 
@@ -22,12 +24,12 @@ namespace {
 
 using at::Tensor;
 
+// A status other than FMOE_OK; becomes fusionllm_amd._lib.FusionMoEError in Python.
+struct StatusError : std::runtime_error {
+  using std::runtime_error::runtime_error;
+};
 [[noreturn]] void raise_status(int rc, const char* what) {
-  py::object err = py::module_::import("fusionllm_amd._lib").attr("FusionMoEError");
-  const std::string msg =
-      std::string(what) + " failed: " + fmoe_status_string(rc) + " (status " + std::to_string(rc) + ")";
-  PyErr_SetString(err.ptr(), msg.c_str());
-  throw py::error_already_set();
+  throw StatusError(std::string(what) + " failed: " + fmoe_status_string(rc) + " (status " + std::to_string(rc) + ")");
 }
 void check(int rc, const char* what) {
   if (rc != FMOE_OK) raise_status(rc, what);
@@ -210,7 +212,15 @@ std::vector<Tensor> backward(const Tensor& dy, const Tensor& x, const Tensor& ga
 
 }  // namespace
 
+// Other Python threads run during a sequence, as they do during a ctypes call.
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
-  m.def("forward", &forward);
-  m.def("backward", &backward);
+  py::register_local_exception_translator([](std::exception_ptr p) {
+    try {
+      if (p) std::rethrow_exception(p);
+    } catch (const StatusError& e) {
+      PyErr_SetString(py::object(py::module_::import("fusionllm_amd._lib").attr("FusionMoEError")).ptr(), e.what());
+    }
+  });
+  m.def("forward", &forward, py::call_guard<py::gil_scoped_release>());
+  m.def("backward", &backward, py::call_guard<py::gil_scoped_release>());
 }

@@ -6,6 +6,7 @@ import torch
 
 from fusionllm_amd import DeepSeekMoE, configs
 from fusionllm_amd import _kernels as K
+from fusionllm_amd._lib import FusionMoEError
 
 pytestmark = pytest.mark.gpu
 
@@ -112,6 +113,15 @@ def test_native_sequence_equals_the_entry_points(gpu_device, T, shared, autocast
     for a, b in zip(*res):
         assert (a is None) == (b is None)
         assert a is None or torch.equal(a, b)
+
+
+def test_native_sequence_reports_refused_shapes(gpu_device):
+    # dim 96 is no multiple of 64: refused on the host, before any launch
+    w, wt = _bf(64, 96, g=None), _bf(96, 64, g=None)
+    x, gw, gb, w1, w2 = (t.to(gpu_device) for t in (_bf(200, 96, g=None), _bf(2, 96, g=None), _bf(2, g=None), w, wt))
+    with pytest.raises(FusionMoEError, match="fmoe_route_and_dispatch"):
+        K.block_host().forward(x, gw, gb, [w1] * 2, [w1] * 2, [w2] * 2, 1, 64, 1.0, False, torch.bfloat16, None, None,
+                               K.stream_handle())
 
 
 @pytest.mark.parametrize("E,k", [(1, 1), (15, 8), (16, 8), (17, 8), (33, 5), (64, 8)])
