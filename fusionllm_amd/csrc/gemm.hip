@@ -1783,9 +1783,32 @@ namespace fmoe {
 // 768, 8 experts 136 -> 81 us, T = 4100 215 -> 185, T = 8192 332 -> 296, C2
 // 500 -> 482 us (one third of the share, rounded up: the left figures; the
 // whole share 532 us at C2, 172 at T = 4100).
-int64_t wgrad_kc(int64_t rows_routed, int64_t rows_shared, int64_t m_out, int64_t n_out) {
+//
+// A launch of one group (a dense layer) knows its rows on the host: it takes
+// the chunk count n with the least rounds * (K steps + 6) + the reduction's
+// n * tiles / 25 + 3 (in K steps' time), so that its n * tiles equal units fill
+// whole rounds of the CUs: 48 tiles of 6100 rows in 8 chunks were 384 units,
+// two rounds of which the second half empty, in 5 they are 240, one round.
+// Forward and backward of the layer, d = 768, I = 2048: T = 6100 311 -> 289 us,
+// T = 9001 454 -> 407, T = 16384 594 -> 547; d = 2048, I = 1408: T = 2048 282 ->
+// 270, T = 6100 460 -> 417, T = 16384 870 -> 850; up to T = 1500 unchanged.
+int64_t wgrad_kc(int64_t rows_routed, int64_t rows_shared, int n_experts, int64_t m_out, int64_t n_out) {
   const int64_t rows = rows_routed + rows_shared;
   const int64_t tiles = ceil_div(m_out, 256) * ceil_div(n_out, 256);
+  if (n_experts == 1 && rows_shared == 0) {
+    const int64_t n_max = (rows + 384) / 768 < 512 ? (rows + 384) / 768 : 512;
+    int64_t best_n = 1, best = 0;
+    for (int64_t n = 1; n <= n_max; ++n) {
+      const int64_t steps = ceil_div(ceil_div(rows, n), 64) + (n > 1 ? 6 : 0);
+      const int64_t cost = ceil_div(n * tiles, 256) * steps * 25 + (n > 1 ? n * tiles + 75 : 0);
+      if (n == 1 || cost < best) {
+        best = cost;
+        best_n = n;
+      }
+    }
+    const int64_t kc = ceil_div(rows, best_n);
+    return kc < 384 ? 384 : kc;
+  }
   const int64_t kc = (tiles * rows / 384) / 64 * 64;
   return kc < 768 ? 768 : kc;
 }
@@ -1794,7 +1817,7 @@ int64_t wgrad_kc(int64_t rows_routed, int64_t rows_shared, int64_t m_out, int64_
 extern "C" size_t fmoe_weight_grad_workspace_bytes(int64_t rows_routed, int64_t rows_shared,
                                                    int n_experts, int64_t m_out, int64_t n_out) {
   if (rows_routed < 0 || rows_shared < 0 || n_experts <= 0 || m_out <= 0 || n_out <= 0) return 0;
-  const int64_t kc = wgrad_kc(rows_routed, rows_shared, m_out, n_out);
+  const int64_t kc = wgrad_kc(rows_routed, rows_shared, n_experts, m_out, n_out);
   // sum over groups of wgrad_chunks(M_g, kc) <= floor(rows / kc) + groups
   const int64_t chunks = (rows_routed + rows_shared) / kc + n_experts + 1;
   return static_cast<size_t>(chunks * m_out * n_out) * sizeof(float);
@@ -1845,7 +1868,7 @@ extern "C" int fmoe_weight_grad(const void* a_routed, const void* a_shared, int6
   a.m_out = static_cast<int>(m_out);
   a.n_out = static_cast<int>(n_out);
   a.m_split = static_cast<int>(m_split);
-  a.kc = static_cast<int>(wgrad_kc(rows_routed, rows_shared, m_out, n_out));
+  a.kc = static_cast<int>(wgrad_kc(rows_routed, rows_shared, n_experts, m_out, n_out));
   a.out_dtype = out_dtype;
   a.partial = static_cast<float*>(workspace);
   const int G = n_experts + (rows_shared > 0 ? 1 : 0);

@@ -67,6 +67,9 @@ def test_row_products_of_small_launches(gpu_device, counts, shared, d, I):
     ([0, 1, 63, 64, 65], 0, 256, 320),       # groups without rows, one stage and its edges
     ([1151, 1152, 1153, 0], 0, 512, 256),    # one chunk or two (kc = 768: from 1152 rows)
     ([100, 2000], 5000, 64, 704),            # shared group in several chunks, a partial tile
+    ([1151], 0, 320, 256),                   # one group: the chunk count that fills whole rounds
+    ([1152], 0, 320, 256),                   # two chunks from here
+    ([5000], 0, 2048, 1536),                 # 48 tiles in five chunks, the last shorter
 ])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_weight_gradient_chunks(gpu_device, counts, shared, m, n, dtype):
