@@ -375,6 +375,17 @@ def gateup_bwd_dx(d_ab, offsets, n_experts: int, rows_routed: int, rows_shared: 
     return dx_rows
 
 
+def _grad_outputs(outs, name, n_groups, numel, dtype):
+    """Addresses of the groups' outputs; the kernel writes numel values of dtype to each."""
+    if len(outs) < n_groups:
+        raise RuntimeError(f"weight_grad needs {n_groups} outputs in {name} (got {len(outs)})")
+    for o in outs:
+        _req(o, name, dtype)
+        if o.numel() != numel:
+            raise RuntimeError(f"{name} must hold {numel} values each (got {tuple(o.shape)})")
+    return ptr_array([o.data_ptr() for o in outs])
+
+
 @_timed
 def weight_grad(a_routed, a_shared, b_routed, b_shared, offsets, n_experts: int, rows_routed: int,
                 rows_shared: int, m_split: int, outs_lo, outs_hi, out_dtype: torch.dtype, b_gather=None,
@@ -387,8 +398,9 @@ def weight_grad(a_routed, a_shared, b_routed, b_shared, offsets, n_experts: int,
     n_out = b_routed.shape[1]
     ws_bytes = lib.fmoe_weight_grad_workspace_bytes(rows_routed, rows_shared, n_experts, m_out, n_out)
     ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=a_routed.device)
-    lo = ptr_array([o.data_ptr() for o in outs_lo])
-    hi = ptr_array([o.data_ptr() for o in outs_hi]) if outs_hi is not None else None
+    G = n_experts + (1 if rows_shared else 0)
+    lo = _grad_outputs(outs_lo, "outs_lo", G, m_split * n_out, out_dtype)
+    hi = None if outs_hi is None else _grad_outputs(outs_hi, "outs_hi", G, (m_out - m_split) * n_out, out_dtype)
     check(lib.fmoe_weight_grad(_req(a_routed, "A", torch.bfloat16),
                                _req(a_shared, "A_shared", torch.bfloat16) if a_shared is not None else None,
                                a_routed.stride(0),

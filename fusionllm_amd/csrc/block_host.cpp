@@ -55,6 +55,14 @@ Tensor empty(at::IntArrayRef shape, at::ScalarType dtype, const Tensor& like) {
   return at::empty(shape, like.options().dtype(dtype).requires_grad(false));
 }
 
+// The dtype in which one launch writes gradients of the dtypes own: theirs if they share it, else
+// fp32, from which each is rounded to its own (the kernel writes every group in one dtype).
+at::ScalarType launch_dtype(const std::vector<at::ScalarType>& own) {
+  for (const at::ScalarType t : own)
+    if (t != own[0]) return at::kFloat;
+  return own[0];
+}
+
 // Addresses of the groups' weights, each checked against its shape.
 std::vector<const void*> weight_ptrs(const std::vector<Tensor>& ws, size_t G, const char* name, int64_t rows,
                                      int64_t cols) {
@@ -179,18 +187,25 @@ std::vector<Tensor> backward(const Tensor& dy, const Tensor& x, const Tensor& ga
                          ws.ptr(), split, s),
         "fmoe_down_bwd_dx");
 
+  std::vector<at::ScalarType> t13, t2;
+  for (size_t g = 0; g < G; ++g) {
+    t13.push_back(grad_dtypes.at(3 * g));
+    t13.push_back(grad_dtypes.at(3 * g + 1));
+    t2.push_back(grad_dtypes.at(3 * g + 2));
+  }
+  const at::ScalarType dt13 = launch_dtype(t13), dt2 = launch_dtype(t2);
   std::vector<Tensor> out(4 + 3 * G);
   std::vector<void*> o1(G), o3(G), o2(G);
   for (size_t g = 0; g < G; ++g) {
-    out[4 + 3 * g] = empty({inter, d}, grad_dtypes.at(3 * g), x);
-    out[5 + 3 * g] = empty({inter, d}, grad_dtypes.at(3 * g + 1), x);
-    out[6 + 3 * g] = empty({d, inter}, grad_dtypes.at(3 * g + 2), x);
+    out[4 + 3 * g] = empty({inter, d}, dt13, x);
+    out[5 + 3 * g] = empty({inter, d}, dt13, x);
+    out[6 + 3 * g] = empty({d, inter}, dt2, x);
     o1[g] = out[4 + 3 * g].data_ptr();
     o3[g] = out[5 + 3 * g].data_ptr();
     o2[g] = out[6 + 3 * g].data_ptr();
   }
   check(fmoe_weight_grad(d_o.data_ptr(), dsp, d, hp, nullptr, inter, nullptr, 1, rows, off, E, rows_r, rows_s, d,
-                         inter, d, o2.data(), nullptr, dtype_code(grad_dtypes.at(2)), ws.ptr(), g2, s),
+                         inter, d, o2.data(), nullptr, dtype_code(dt2), ws.ptr(), g2, s),
         "fmoe_weight_grad");
   out[0] = empty({rows, d}, bf, x);
   check(fmoe_gateup_bwd_dx(d_ab.data_ptr(), off, E, rows_r, rows_s, d, inter, p1.data(), p3.data(),
@@ -198,7 +213,7 @@ std::vector<Tensor> backward(const Tensor& dy, const Tensor& x, const Tensor& ga
         "fmoe_gateup_bwd_dx");
   check(fmoe_weight_grad(d_ab.data_ptr(), nullptr, 2 * inter, xpp, has_shared ? xp : nullptr, d, nullptr, 1, rows_r,
                          off, E, rows_r, rows_s, 2 * inter, d, inter, o1.data(), o3.data(),
-                         dtype_code(grad_dtypes.at(0)), ws.ptr(), g13, s),
+                         dtype_code(dt13), ws.ptr(), g13, s),
         "fmoe_weight_grad");
   out[1] = empty({T, k}, at::kFloat, x);
   out[2] = empty({E, d}, gate_grad_dtype, x);
@@ -207,6 +222,8 @@ std::vector<Tensor> backward(const Tensor& dy, const Tensor& x, const Tensor& ga
                         d, E, kk, rs, static_cast<float*>(out[1].data_ptr()), out[2].data_ptr(), out[3].data_ptr(),
                         dtype_code(gate_grad_dtype), ws.ptr(), rb, s),
         "fmoe_router_bwd");
+  for (size_t i = 0; i < 3 * G; ++i)
+    if (out[4 + i].scalar_type() != grad_dtypes[i]) out[4 + i] = out[4 + i].to(grad_dtypes[i]);
   return out;
 }
 

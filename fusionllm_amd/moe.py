@@ -357,18 +357,29 @@ def _backward_pass(ctx, saved, dy):
     # Down projection: dX with the SwiGLU backward fused (reading w2 as it
     # lies), then dW2.
     d_ab = K.down_bwd_dx(d_o, dy_sh, offsets, E, w2s, ab, inter)
-    dw2 = [torch.empty(d, inter, dtype=w_dtypes[3 * g + 2], device=xb.device) for g in range(G)]
-    K.weight_grad(d_o, dy_sh, h, None, offsets, E, rows_r, rows_s, d, dw2, None,
-                  w_dtypes[2], tag="w2")
+    t1, t3, t2 = (w_dtypes[i:3 * G:3] for i in range(3))
+    dt2 = _launch_dtype(t2)
+    dw2 = [torch.empty(d, inter, dtype=dt2, device=xb.device) for g in range(G)]
+    K.weight_grad(d_o, dy_sh, h, None, offsets, E, rows_r, rows_s, d, dw2, None, dt2, tag="w2")
     # Gate/up projections: dX (one product over [w1; w3]) then dW1, dW3.
     dx_rows = K.gateup_bwd_dx(d_ab, offsets, E, rows_r, rows_s, w1s, w3s, d)
-    dw1 = [torch.empty(inter, d, dtype=w_dtypes[3 * g], device=xb.device) for g in range(G)]
-    dw3 = [torch.empty(inter, d, dtype=w_dtypes[3 * g + 1], device=xb.device) for g in range(G)]
+    dt13 = _launch_dtype([*t1, *t3])
+    dw1 = [torch.empty(inter, d, dtype=dt13, device=xb.device) for g in range(G)]
+    dw3 = [torch.empty(inter, d, dtype=dt13, device=xb.device) for g in range(G)]
     K.weight_grad(d_ab, None, xb if gather else x_perm, xb if has_shared else None, offsets, E, rows_r, rows_s,
-                  inter, dw1, dw3, w_dtypes[0], b_gather=perm if gather else None, k=k, tag="w13")
+                  inter, dw1, dw3, dt13, b_gather=perm if gather else None, k=k, tag="w13")
     # Router: logits gradient, gate weight/bias gradient.
     d_logits, dgw, dgb = K.router_bwd(d_w, v, perm, offsets, xb, E, rs, gw_dtype)
+    dw1, dw3, dw2 = ([g if g.dtype == t else g.to(t) for g, t in zip(gs, ts)]
+                     for gs, ts in ((dw1, t1), (dw3, t3), (dw2, t2)))
     return dx_rows, d_logits, dgw, _gate_bias_grad(dgb, gb_dtype), _expert_grads(ctx, dw1, dw3, dw2, wb)
+
+
+def _launch_dtype(dtypes):
+    """The dtype in which one weight-gradient launch writes gradients of these
+    dtypes (autocast takes mixed parameters): theirs if they share it, else
+    fp32, from which each is rounded to its own."""
+    return dtypes[0] if len(set(dtypes)) == 1 else torch.float32
 
 
 def _gate_bias_grad(dgb, dtype):

@@ -146,3 +146,58 @@ def test_topk_ties_and_nan_across_lanes(gpu_device, E, k):
     keep[3] = False
     assert torch.equal(got[keep], want.expand(T - 1, k))
     assert torch.equal(got[3], torch.arange(k)) and torch.isnan(v[3]).all()
+
+
+def _mixed(m, which):
+    """bf16 for some of an fp32 module's parameters (autocast takes any mix)."""
+    for n, p in m.named_parameters():
+        if {"shared": n.startswith("shared_expert"), "w3": n.endswith("w3.weight"),
+            "w1, a w2": n.endswith("w1.weight") or n == "experts.2.w2.weight",
+            "first expert": n.startswith("experts.0.")}[which]:
+            p.data = p.data.bfloat16()
+    return m
+
+
+@pytest.mark.parametrize("which", ["shared", "w3", "w1, a w2", "first expert"])
+@pytest.mark.parametrize("path", ["native", "wrappers", "operator"])
+def test_weight_gradients_of_mixed_parameter_dtypes(gpu_device, which, path):
+    # The values are bf16 ones, so the kernels read the same operands whatever
+    # the parameters' dtypes: each gradient is the fp32 module's, rounded once
+    # to its parameter's dtype.
+    cfg = configs.BlockConfig("mixed", 300, dim=128, inter=192, n_experts=4, topk=2, n_shared=1, bias="skew")
+    data = configs.make_block(cfg, seed=9)
+    grads = []
+    for mixed in (False, True):
+        m = DeepSeekMoE(cfg.moe_config())
+        m.load_state_dict({n: t.bfloat16().float() for n, t in data.state_dict().items()})
+        m = m.to(gpu_device, torch.float32)
+        m = _mixed(m, which) if mixed else m
+        x = data.x.to(gpu_device).bfloat16().float()
+        K.set_timer({} if path == "wrappers" else None)
+        try:
+            with torch.autocast("cuda", dtype=torch.bfloat16):
+                if path == "operator":
+                    y = torch.ops.fusionllm.moe_fwd(x, m.gate.weight, m.gate.bias, m._flat_weights(), 2, 1.0, True,
+                                                    torch.float32)[0]
+                else:
+                    y = m(x)
+            y.backward(data.dy.to(gpu_device, y.dtype))
+        finally:
+            K.set_timer(None)
+        grads.append({n: (p.dtype, p.grad) for n, p in m.named_parameters()})
+    assert len({t for t, _ in grads[1].values()}) == 2
+    for n, (t, got) in grads[1].items():
+        want = grads[0][n][1]
+        assert (got is None) == (want is None), n
+        assert got is None or (got.dtype == t and torch.equal(got, want.to(t))), n
+
+
+def test_weight_grad_refuses_outputs_that_do_not_fit(gpu_device):
+    # on the host, before the launch
+    off, rr = _groups([64, 64], gpu_device)
+    a, b = (torch.zeros(rr, n, dtype=torch.bfloat16, device=gpu_device) for n in (128, 64))
+    out = lambda *s, dtype=torch.float32: torch.empty(*s, dtype=dtype, device=gpu_device)
+    for outs in ([out(128, 64), out(128, 64, dtype=torch.bfloat16)], [out(128, 64), out(64, 64)], [out(128, 64)],
+                 [out(128, 64), out(64, 128).t()]):
+        with pytest.raises(RuntimeError, match="outs_lo"):
+            K.weight_grad(a, None, b, None, off, 2, rr, 0, 128, outs, None, torch.float32)
