@@ -1142,12 +1142,16 @@ __global__ __launch_bounds__(core::NT, 1) void wgrad_tr_kernel(const WgradArgs a
                                                                const int32_t* __restrict__ offsets) {
   using namespace core;
   __shared__ __attribute__((aligned(1024))) uint8_t smem[2 * STAGE];
-  // Gathered B rows: the slot indices of each stage's 64 k rows (ring of eight
-  // stages, filled by global -> LDS copies three stages ahead of a stage's
-  // copies and read when its first B unit is issued, after waits that cover
-  // them; a slot is refilled stages after its last read, with barriers in
-  // between).
-  __shared__ int32_t idx_ring[8][BK];
+  // Gathered B rows: the slot indices of each stage's 64 k rows, a ring of eight
+  // stages per wave, so that every wave issues the same operations and the
+  // waits can count them (of one ring that wave 0 fills they can't, and waiting
+  // for all copies instead drains the ring of stages every step: dW1|dW3 823
+  // -> 350 us at C2, 5500 -> 2549 at C5, 622 -> 308 at T = 9001, d = 1024, I = 1536,
+  // 16 experts; with the rows copied beforehand 335, 2392 and 290).  Filled by
+  // global -> LDS copies three stages ahead of a stage's copies and read when
+  // its first B unit is issued, by the wave that filled it, after a wait that
+  // covers them; a slot is refilled stages after its last read.
+  __shared__ int32_t idx_ring[GATHER ? 8 : 1][8][BK];
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = w / WN, wn = w % WN;  // wave block: 64 m x 128 n
@@ -1214,14 +1218,15 @@ __global__ __launch_bounds__(core::NT, 1) void wgrad_tr_kernel(const WgradArgs a
                       : gathered ? args.b_routed
                                  : args.b_routed + static_cast<int64_t>(row_base) * args.ldb;
   const int lda = static_cast<int>(args.lda), ldb = static_cast<int>(args.ldb);
-  const uint32_t ring = lds_addr(&idx_ring[0][0]);
-  // stage kt's slot indices into ring slot kt % 8 (wave 0; rows past k_end
-  // repeat the last valid one)
+  const int wr = GATHER ? w : 0;
+  const uint32_t ring = lds_addr(&idx_ring[wr][0][0]);
+  // stage kt's slot indices into ring slot kt % 8 (rows past k_end repeat the
+  // last valid one; the shared group, whose rows are not gathered, fetches a
+  // value that it does not use, so that its count is the same)
+  const int32_t* idx_src = gathered ? args.b_gather + row_base : offsets;
   auto fetch_idx = [&](int kt) {
-    if (w == 0) {
-      const int r = min(k_begin + kt * BK + lane, k_end - 1);
-      copy4(ring + (kt & 7) * (BK * 4), args.b_gather + row_base, static_cast<uint32_t>(r) * 4u);
-    }
+    const int r = gathered ? min(k_begin + kt * BK + lane, k_end - 1) : 0;
+    copy4(ring + (kt & 7) * (BK * 4), idx_src, static_cast<uint32_t>(r) * 4u);
   };
   // ---- copies: a unit is 128 columns of a stage's 64 k rows (A0, A1, B0, B1
   // in LDS); instruction i of wave w writes its k rows 32 i + drow (1 KB = 4
@@ -1233,7 +1238,7 @@ __global__ __launch_bounds__(core::NT, 1) void wgrad_tr_kernel(const WgradArgs a
   if (gathered) {
     // stages 0..2 before the first copies (stage kt's last unit fetches stage kt + 3)
     for (int q = 0; q < 3 && q < nk; ++q) fetch_idx(q);
-    asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
 
   // Unit u of a stage (two instructions); a stage's units are issued in the
@@ -1262,7 +1267,7 @@ __global__ __launch_bounds__(core::NT, 1) void wgrad_tr_kernel(const WgradArgs a
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int r = min(32 * i + drow, last);
-      const uint32_t tok = slot_token(static_cast<uint32_t>(idx_ring[kt & 7][r]), args.gather_magic);
+      const uint32_t tok = slot_token(static_cast<uint32_t>(idx_ring[wr][kt & 7][r]), args.gather_magic);
 #pragma unroll
       for (int u = 0; u < 2; ++u)
         b_off[2 * u + i] = (tok * static_cast<uint32_t>(ldb) +
@@ -1274,7 +1279,7 @@ __global__ __launch_bounds__(core::NT, 1) void wgrad_tr_kernel(const WgradArgs a
 #pragma unroll
     for (int i = 0; i < 2; ++i) copy16(lds_copy + (kt & 1) * STAGE + u * UNIT + i * 8192, pa, a_off[2 * u + i]);
     if (u == 0) return;
-    if (GATHER && gathered && kt + 3 < nk) fetch_idx(kt + 3);
+    if (GATHER) fetch_idx(kt + 3);
     if (kt + 1 < nk) {
       pa += 2 * BK * args.lda;
       if (!gathered) pb += 2 * BK * args.ldb;
@@ -1296,12 +1301,16 @@ __global__ __launch_bounds__(core::NT, 1) void wgrad_tr_kernel(const WgradArgs a
     for (int i = 0; i < 2; ++i)
       if (k0 + 32 * i + drow >= k_end) *reinterpret_cast<uint4*>(st + i * 8192) = make_uint4(0, 0, 0, 0);
   };
-  // All but the N newest copies of this wave have landed (the gathered rows'
-  // index fetches make wave 0's count differ, so that variant waits for all).
-  auto wait_copies = [&](auto n) {
-    if (GATHER) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(decltype(n)::value) : "memory");
+  // All but the newest copies of this wave have landed: those of UNITS units,
+  // and the FETCHES index fetches among them (one follows each A1).
+  auto wait_copies = [&](auto units, auto fetches) {
+    constexpr int N = decltype(units)::value * LU + (GATHER ? decltype(fetches)::value : 0);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
   };
+  constexpr std::integral_constant<int, 1> n1{};
+  constexpr std::integral_constant<int, 2> n2{};
+  constexpr std::integral_constant<int, 4> n4{};
+  constexpr std::integral_constant<int, 5> n5{};
 
   // ---- fragment addresses within a unit: the wave's 32 A columns (2 windows), 64 B columns (4)
   uint32_t xa = tr_base(2 * wm, lane), xb = A_BYTES + tr_base(4 * wn, lane);
@@ -1334,7 +1343,7 @@ __global__ __launch_bounds__(core::NT, 1) void wgrad_tr_kernel(const WgradArgs a
     issue_a(1, 0);
     issue_b(1, 0);
     issue_b(1, 1);
-    wait_copies(std::integral_constant<int, 5 * LU>{});
+    wait_copies(n5, n1);  // A0, B0 of stage 0
     zero_tail(0, 0);
     wait_lds_barrier();
     read_first(sbase);
@@ -1348,7 +1357,7 @@ __global__ __launch_bounds__(core::NT, 1) void wgrad_tr_kernel(const WgradArgs a
 #pragma unroll
       for (int n = 0; n < 4; ++n) read_b(b0, cur, 1, n);
       issue_a(kt + 1, 1);
-      wait_copies(std::integral_constant<int, 5 * LU>{});  // B1 of this stage
+      wait_copies(n5, n2);  // B1 of this stage
       wait_lds_barrier();
       quarter<0, 0>(acc, a0, b0);
       // (0, 1)
@@ -1357,7 +1366,7 @@ __global__ __launch_bounds__(core::NT, 1) void wgrad_tr_kernel(const WgradArgs a
 #pragma unroll
         for (int n = 0; n < 4; ++n) read_b(b1, cur + UNIT, kh, n);
       issue_a(kt + 2, 0);
-      wait_copies(std::integral_constant<int, 5 * LU>{});  // A1 of this stage
+      wait_copies(n5, n2);  // A1 of this stage (its own fetch may be in flight)
       zero_tail(kt, 1);
       wait_lds_barrier();
       quarter<0, 1>(acc, a0, b1);
@@ -1369,7 +1378,7 @@ __global__ __launch_bounds__(core::NT, 1) void wgrad_tr_kernel(const WgradArgs a
       // gathered B: the offsets of stage kt + 2, whose ring slot landed a step ago
       if (gathered) form_gathered(min(kt + 2, nk - 1));
       issue_b(kt + 2, 0);
-      wait_copies(std::integral_constant<int, 4 * LU>{});  // A0, B0 of the next stage
+      wait_copies(n4, n1);  // A0, B0 of the next stage
       zero_tail(kt + 1, 0);
       wait_lds_barrier();
       quarter<1, 0>(acc, a1, b0);

@@ -223,8 +223,9 @@ class DenseFFN(SwiGLUExpert):
 # instead of writing the gathered copy x_perm.  Measured on one MI355X at C2
 # (16384 tokens, both variants in one session): dropping the copy saves 11 us
 # in the dispatch, but the gate/up forward reading rows through perm takes
-# 9-14 us longer and dW1|dW3 18-21 us longer (scattered 128-byte row pieces
-# instead of consecutive rows), so the block keeps x_perm.  The entry points
+# 5-10 us longer (305 against 300) and dW1|dW3 15 us longer (350 against 335;
+# scattered 128-byte row pieces instead of consecutive rows), so the block
+# keeps x_perm.  The entry points
 # keep the option (fmoe_gateup_fwd, fmoe_weight_grad): it saves T*k*dim*2
 # bytes of HBM.
 GATHER_ROWS = False

@@ -201,3 +201,24 @@ def test_weight_grad_refuses_outputs_that_do_not_fit(gpu_device):
                  [out(128, 64), out(64, 128).t()]):
         with pytest.raises(RuntimeError, match="outs_lo"):
             K.weight_grad(a, None, b, None, off, 2, rr, 0, 128, outs, None, torch.float32)
+
+
+@pytest.mark.parametrize("counts,shared,m,n", [
+    ([0, 1, 63, 64, 65], 0, 256, 320),        # one stage of 64 rows and its edges
+    ([127, 129, 192, 193, 255], 300, 64, 64),  # two to four stages: fewer than are fetched ahead; a shared group
+    ([512, 513, 577, 4000], 1100, 320, 576),   # past the eight stages of the index ring, several chunks
+])
+def test_gathered_weight_gradient_equals_the_copied_rows(gpu_device, counts, shared, m, n):
+    D = gpu_device
+    g = torch.Generator().manual_seed(sum(counts))
+    E, G = len(counts), len(counts) + (1 if shared else 0)
+    off, rr = _groups(counts, D)
+    T, k = (rr + 2) // 3, 3
+    x, a = _bf(T, n, g=g).to(D), _bf(rr, m, g=g).to(D)
+    perm = torch.randperm(T * k, generator=g)[:rr].to(torch.int32).to(D)
+    sa, sb = (_bf(shared, m, g=g).to(D), _bf(shared, n, g=g).to(D)) if shared else (None, None)
+    outs = [[torch.full((m, n), float("nan"), device=D) for _ in range(G)] for _ in range(2)]
+    K.weight_grad(a, sa, x[perm.long() // k].contiguous(), sb, off, E, rr, shared, m, outs[0], None, torch.float32)
+    K.weight_grad(a, sa, x, sb, off, E, rr, shared, m, outs[1], None, torch.float32, b_gather=perm, k=k)
+    for want, got in zip(*outs):
+        assert torch.equal(want, got)
