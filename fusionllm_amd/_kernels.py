@@ -72,12 +72,14 @@ def block_host():
     if _TIMER is not None:
         return None
     if _BLOCK_HOST is None:
-        _lib.load()
+        lib = _lib.load()
         try:
             from . import _block_host
         except ImportError as e:
             raise FileNotFoundError("fusionllm_amd/_block_host.so is missing or does not load: build the extension "
                                     "first (python -m fusionllm_amd.build or __graft_entry__.build())") from e
+        _block_host.bind([ctypes.cast(getattr(lib, name), ctypes.c_void_p).value
+                          for name in _block_host.entry_points()])
         _BLOCK_HOST = _block_host
     return _BLOCK_HOST
 

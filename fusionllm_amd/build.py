@@ -13,6 +13,7 @@ module _block_host beside it.  Compiler flags of the kernels:
 """
 from __future__ import annotations
 
+import importlib.util
 import os
 import subprocess
 import sys
@@ -53,8 +54,9 @@ def _compile(src: Path) -> Path:
 
 
 def build_host_module() -> Path:
-    """Compile csrc/block_host.cpp (the block's launch sequence on torch's C++ API,
-    linked against libfusionmoe.so next to it) into the module _block_host."""
+    """Compile csrc/block_host.cpp (the block's launch sequence on torch's C++ API;
+    it is given the entry points of the loaded library at run time) into the
+    module _block_host."""
     import sysconfig
 
     import torch
@@ -67,8 +69,7 @@ def build_host_module() -> Path:
            "-DTORCH_EXTENSION_NAME=_block_host",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
            *[f"-I{i}" for i in includes], str(CSRC / "block_host.cpp"), "-o", str(tmp),
-           f"-L{PKG_DIR}", "-lfusionmoe", f"-L{libdir}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10",
-           "-Wl,-rpath,$ORIGIN"]
+           f"-L{libdir}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10"]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"{cmd[0]} failed on block_host.cpp:\n{res.stdout}\n{res.stderr}")
@@ -77,8 +78,9 @@ def build_host_module() -> Path:
 
 
 def build_library(verbose: bool = True) -> Path:
-    """Compile every kernel source, link libfusionmoe.so and build the host module on it;
-    returns the library's path."""
+    """Compile every kernel source and link libfusionmoe.so; where torch is installed, build
+    the host module too (the library and its C ABI need neither torch nor a host compiler).
+    Returns the library's path."""
     BUILD_DIR.mkdir(exist_ok=True)
     sources = sorted(CSRC.glob("*.hip"))
     if not sources:
@@ -91,7 +93,8 @@ def build_library(verbose: bool = True) -> Path:
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stdout}\n{res.stderr}")
     os.replace(tmp, LIB_PATH)
-    build_host_module()
+    if importlib.util.find_spec("torch") is not None:
+        build_host_module()
     if verbose:
         print(f"built {LIB_PATH} from {len(sources)} sources", file=sys.stderr)
     return LIB_PATH

@@ -24,12 +24,45 @@ namespace {
 
 using at::Tensor;
 
+// The entry points of the library that fusionllm_amd._lib loaded (bind), so
+// that a program which chose another build of it launches that one here too.
+#define FMOE_ENTRY_POINTS(F)                                                                              \
+  F(fmoe_status_string) F(fmoe_split_workspace_bytes) F(fmoe_route_and_dispatch_workspace_bytes)          \
+  F(fmoe_route_and_dispatch) F(fmoe_gateup_fwd) F(fmoe_down_fwd) F(fmoe_combine_fwd) F(fmoe_combine_bwd)  \
+  F(fmoe_down_bwd_dx) F(fmoe_weight_grad_workspace_bytes) F(fmoe_weight_grad) F(fmoe_gateup_bwd_dx)       \
+  F(fmoe_router_bwd_workspace_bytes) F(fmoe_router_bwd)
+struct Api {
+#define F(name) decltype(&::name) name = nullptr;
+  FMOE_ENTRY_POINTS(F)
+#undef F
+} api;
+
+// Names of the entry points used here.
+std::vector<std::string> entry_points() {
+#define F(name) #name,
+  return {FMOE_ENTRY_POINTS(F)};
+#undef F
+}
+
+// Their addresses, in that order.
+void bind(const std::vector<uint64_t>& addresses) {
+  if (addresses.size() != entry_points().size()) throw std::runtime_error("one address per entry point is needed");
+  size_t i = 0;
+#define F(name) api.name = reinterpret_cast<decltype(api.name)>(addresses[i++]);
+  FMOE_ENTRY_POINTS(F)
+#undef F
+}
+
+void need_entry_points() {
+  if (api.fmoe_status_string == nullptr) throw std::runtime_error("bind() has not been called");
+}
+
 // A status other than FMOE_OK; becomes fusionllm_amd._lib.FusionMoEError in Python.
 struct StatusError : std::runtime_error {
   using std::runtime_error::runtime_error;
 };
 [[noreturn]] void raise_status(int rc, const char* what) {
-  throw StatusError(std::string(what) + " failed: " + fmoe_status_string(rc) + " (status " + std::to_string(rc) + ")");
+  throw StatusError(std::string(what) + " failed: " + api.fmoe_status_string(rc) + " (status " + std::to_string(rc) + ")");
 }
 void check(int rc, const char* what) {
   if (rc != FMOE_OK) raise_status(rc, what);
@@ -98,6 +131,7 @@ std::vector<Tensor> forward(const Tensor& x, const Tensor& gate_w, const Tensor&
                             const std::vector<Tensor>& w2, int64_t k, int64_t inter, double route_scale,
                             bool has_shared, at::ScalarType out_dtype, const c10::optional<Tensor>& residual,
                             const c10::optional<Tensor>& counts_host, uint64_t stream) {
+  need_entry_points();
   void* s = reinterpret_cast<void*>(stream);
   const int64_t T = x.size(0), d = x.size(1);
   const int E = static_cast<int>(gate_w.size(0));
@@ -118,10 +152,10 @@ std::vector<Tensor> forward(const Tensor& x, const Tensor& gate_w, const Tensor&
       throw std::runtime_error("counts_host must be a contiguous pinned int32 CPU tensor of n_experts elements");
     ch = c.data_ptr();
   }
-  const size_t split = fmoe_split_workspace_bytes();
-  const size_t rd = fmoe_route_and_dispatch_workspace_bytes(T, E, kk);
+  const size_t split = api.fmoe_split_workspace_bytes();
+  const size_t rd = api.fmoe_route_and_dispatch_workspace_bytes(T, E, kk);
   const Workspace ws(std::max(split, rd), x);
-  check(fmoe_route_and_dispatch(xp, gwp, gbp, T, d, E, kk, static_cast<float>(route_scale),
+  check(api.fmoe_route_and_dispatch(xp, gwp, gbp, T, d, E, kk, static_cast<float>(route_scale),
                                 static_cast<int32_t*>(idx.data_ptr()), static_cast<int64_t*>(idx64.data_ptr()),
                                 static_cast<float*>(w.data_ptr()), static_cast<float*>(v.data_ptr()),
                                 static_cast<int32_t*>(counts.data_ptr()), static_cast<int32_t*>(offsets.data_ptr()),
@@ -130,15 +164,15 @@ std::vector<Tensor> forward(const Tensor& x, const Tensor& gate_w, const Tensor&
         "fmoe_route_and_dispatch");
   const int32_t* off = static_cast<const int32_t*>(offsets.data_ptr());
   Tensor ab = empty({rows, 2 * inter}, bf, x), h = empty({rows, inter}, bf, x);
-  check(fmoe_gateup_fwd(x_perm.data_ptr(), nullptr, kk, rows_r, has_shared ? xp : nullptr, off, E, rows_r, rows_s, d,
+  check(api.fmoe_gateup_fwd(x_perm.data_ptr(), nullptr, kk, rows_r, has_shared ? xp : nullptr, off, E, rows_r, rows_s, d,
                         inter, p1.data(), p3.data(), ab.data_ptr(), h.data_ptr(), ws.ptr(), split, s),
         "fmoe_gateup_fwd");
   Tensor o = empty({rows, d}, bf, x);
-  check(fmoe_down_fwd(h.data_ptr(), off, E, rows_r, rows_s, d, inter, p2.data(), o.data_ptr(), ws.ptr(), split, s),
+  check(api.fmoe_down_fwd(h.data_ptr(), off, E, rows_r, rows_s, d, inter, p2.data(), o.data_ptr(), ws.ptr(), split, s),
         "fmoe_down_fwd");
   Tensor y = empty({T, d}, out_dtype, x);
   const void* res = residual.has_value() ? req(*residual, "residual", out_dtype) : nullptr;
-  check(fmoe_combine_fwd(o.data_ptr(), static_cast<int32_t*>(idx.data_ptr()), static_cast<float*>(w.data_ptr()),
+  check(api.fmoe_combine_fwd(o.data_ptr(), static_cast<int32_t*>(idx.data_ptr()), static_cast<float*>(w.data_ptr()),
                          static_cast<int32_t*>(pos.data_ptr()), T, d, kk, rows_r, has_shared, dtype_code(out_dtype),
                          res, y.data_ptr(), s),
         "fmoe_combine_fwd");
@@ -154,6 +188,7 @@ std::vector<Tensor> backward(const Tensor& dy, const Tensor& x, const Tensor& ga
                              const std::vector<Tensor>& w3, const std::vector<Tensor>& w2, int64_t k, int64_t inter,
                              double route_scale, bool has_shared, at::ScalarType gate_grad_dtype,
                              const std::vector<at::ScalarType>& grad_dtypes, uint64_t stream) {
+  need_entry_points();
   void* s = reinterpret_cast<void*>(stream);
   const int64_t T = x.size(0), d = x.size(1);
   const int E = static_cast<int>(gate_w.size(0));
@@ -170,20 +205,20 @@ std::vector<Tensor> backward(const Tensor& dy, const Tensor& x, const Tensor& ga
              *xpp = req(x_perm, "x_perm", bf), *vp = req(v, "topv", at::kFloat);
   const int32_t* off = static_cast<const int32_t*>(offp);
   const int32_t* permp = static_cast<const int32_t*>(pp);
-  const size_t split = fmoe_split_workspace_bytes();
-  const size_t g2 = fmoe_weight_grad_workspace_bytes(rows_r, rows_s, E, d, inter);
-  const size_t g13 = fmoe_weight_grad_workspace_bytes(rows_r, rows_s, E, 2 * inter, d);
-  const size_t rb = fmoe_router_bwd_workspace_bytes(T, d, E, kk);
+  const size_t split = api.fmoe_split_workspace_bytes();
+  const size_t g2 = api.fmoe_weight_grad_workspace_bytes(rows_r, rows_s, E, d, inter);
+  const size_t g13 = api.fmoe_weight_grad_workspace_bytes(rows_r, rows_s, E, 2 * inter, d);
+  const size_t rb = api.fmoe_router_bwd_workspace_bytes(T, d, E, kk);
   const Workspace ws(std::max(std::max(split, rb), std::max(g2, g13)), x);
 
   Tensor d_o = empty({rows_r, d}, bf, x), d_w = empty({T, k}, at::kFloat, x);
-  check(fmoe_combine_bwd(dyp, dtype_code(dy.scalar_type()), op, static_cast<const float*>(wp), permp, T, d, kk,
+  check(api.fmoe_combine_bwd(dyp, dtype_code(dy.scalar_type()), op, static_cast<const float*>(wp), permp, T, d, kk,
                          d_o.data_ptr(), static_cast<float*>(d_w.data_ptr()), s),
         "fmoe_combine_bwd");
   Tensor dy_sh = has_shared ? dy.to(bf).contiguous() : Tensor();
   const void* dsp = has_shared ? dy_sh.data_ptr() : nullptr;
   Tensor d_ab = empty({rows, 2 * inter}, bf, x);
-  check(fmoe_down_bwd_dx(d_o.data_ptr(), dsp, off, E, rows_r, rows_s, d, inter, p2.data(), abp, d_ab.data_ptr(),
+  check(api.fmoe_down_bwd_dx(d_o.data_ptr(), dsp, off, E, rows_r, rows_s, d, inter, p2.data(), abp, d_ab.data_ptr(),
                          ws.ptr(), split, s),
         "fmoe_down_bwd_dx");
 
@@ -204,21 +239,21 @@ std::vector<Tensor> backward(const Tensor& dy, const Tensor& x, const Tensor& ga
     o3[g] = out[5 + 3 * g].data_ptr();
     o2[g] = out[6 + 3 * g].data_ptr();
   }
-  check(fmoe_weight_grad(d_o.data_ptr(), dsp, d, hp, nullptr, inter, nullptr, 1, rows, off, E, rows_r, rows_s, d,
+  check(api.fmoe_weight_grad(d_o.data_ptr(), dsp, d, hp, nullptr, inter, nullptr, 1, rows, off, E, rows_r, rows_s, d,
                          inter, d, o2.data(), nullptr, dtype_code(dt2), ws.ptr(), g2, s),
         "fmoe_weight_grad");
   out[0] = empty({rows, d}, bf, x);
-  check(fmoe_gateup_bwd_dx(d_ab.data_ptr(), off, E, rows_r, rows_s, d, inter, p1.data(), p3.data(),
+  check(api.fmoe_gateup_bwd_dx(d_ab.data_ptr(), off, E, rows_r, rows_s, d, inter, p1.data(), p3.data(),
                            out[0].data_ptr(), ws.ptr(), split, s),
         "fmoe_gateup_bwd_dx");
-  check(fmoe_weight_grad(d_ab.data_ptr(), nullptr, 2 * inter, xpp, has_shared ? xp : nullptr, d, nullptr, 1, rows_r,
+  check(api.fmoe_weight_grad(d_ab.data_ptr(), nullptr, 2 * inter, xpp, has_shared ? xp : nullptr, d, nullptr, 1, rows_r,
                          off, E, rows_r, rows_s, 2 * inter, d, inter, o1.data(), o3.data(),
                          dtype_code(dt13), ws.ptr(), g13, s),
         "fmoe_weight_grad");
   out[1] = empty({T, k}, at::kFloat, x);
   out[2] = empty({E, d}, gate_grad_dtype, x);
   out[3] = empty({E}, gate_grad_dtype, x);
-  check(fmoe_router_bwd(static_cast<const float*>(d_w.data_ptr()), static_cast<const float*>(vp), permp, off, xp, T,
+  check(api.fmoe_router_bwd(static_cast<const float*>(d_w.data_ptr()), static_cast<const float*>(vp), permp, off, xp, T,
                         d, E, kk, rs, static_cast<float*>(out[1].data_ptr()), out[2].data_ptr(), out[3].data_ptr(),
                         dtype_code(gate_grad_dtype), ws.ptr(), rb, s),
         "fmoe_router_bwd");
@@ -238,6 +273,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
       PyErr_SetString(py::object(py::module_::import("fusionllm_amd._lib").attr("FusionMoEError")).ptr(), e.what());
     }
   });
+  m.def("entry_points", &entry_points);
+  m.def("bind", &bind);
   m.def("forward", &forward, py::call_guard<py::gil_scoped_release>());
   m.def("backward", &backward, py::call_guard<py::gil_scoped_release>());
 }

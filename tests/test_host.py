@@ -397,3 +397,57 @@ def test_operator_fake_shapes():
         assert len(g) == 3 + len(ws)
         assert (tuple(g[0].shape), g[0].dtype) == ((T, d), torch.float32)
         assert all(tuple(a.shape) == tuple(b.shape) for a, b in zip(g[3:], ws))
+
+
+def test_a_chosen_library_serves_the_native_sequences_too(tmp_path):
+    # _lib.load(path) selects the library for every call of the process: the
+    # native module gets its entry points and brings no other library in.
+    import shutil
+    import subprocess
+    import sys
+    other = tmp_path / "libfusionmoe_other.so"
+    shutil.copy(_lib.LIB_PATH, other)
+    code = f"""
+from fusionllm_amd import _kernels, _lib
+_lib.load({str(other)!r})
+host = _kernels.block_host()
+assert "fmoe_gateup_fwd" in host.entry_points()
+maps = open("/proc/self/maps").read()
+assert {str(other)!r} in maps
+assert {str(_lib.LIB_PATH)!r} not in maps, "the library beside the package was loaded as well"
+"""
+    res = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=300)
+    assert res.returncode == 0, res.stderr
+
+
+def test_native_module_without_entry_points_raises(tmp_path):
+    import subprocess
+    import sys
+    code = """
+import torch
+from fusionllm_amd import _block_host
+t = torch.empty(1, 1)
+try:
+    _block_host.forward(t, t, t, [], [], [], 1, 64, 1.0, False, torch.bfloat16, None, None, 0)
+except RuntimeError as e:
+    assert "bind" in str(e), e
+else:
+    raise AssertionError("no error")
+"""
+    res = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=300)
+    assert res.returncode == 0, res.stderr
+
+
+def test_build_library_needs_no_torch(monkeypatch):
+    # Where torch is not installed, the kernel library is built alone.
+    from fusionllm_amd import build
+    ran = []
+    monkeypatch.setattr(build, "_compile", lambda src: Path("/dev/null"))
+    monkeypatch.setattr(build.subprocess, "run", lambda cmd, **kw: type("R", (), {"returncode": 0})())
+    monkeypatch.setattr(build.os, "replace", lambda a, b: None)
+    monkeypatch.setattr(build, "build_host_module", lambda: ran.append(1))
+    for spec, n in ((None, 0), (object(), 1)):
+        ran.clear()
+        monkeypatch.setattr(build.importlib.util, "find_spec", lambda name: spec)
+        build.build_library(verbose=False)
+        assert len(ran) == n
