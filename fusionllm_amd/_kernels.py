@@ -244,7 +244,7 @@ def gateup_fwd(x_rows, x_shared, offsets, n_experts: int, w1s, w3s, inter: int, 
     rows = rows_r + rows_s
     ab = torch.empty(rows, 2 * inter, dtype=torch.bfloat16, device=dev)
     h = torch.empty(rows, inter, dtype=torch.bfloat16, device=dev)
-    ws, ws_bytes = _split_workspace(dev, rows_r, rows_s, -(-inter // 128), small=True)
+    ws, ws_bytes = _split_workspace(dev, rows_r, rows_s, d, -(-inter // 128), small=True)
     check(lib.fmoe_gateup_fwd(_req(x_rows, "x_rows", torch.bfloat16),
                               _req(gather, "gather", torch.int32) if gather is not None else None, int(k),
                               x_rows.shape[0],
@@ -258,6 +258,7 @@ def gateup_fwd(x_rows, x_shared, offsets, n_experts: int, w1s, w3s, inter: int, 
 
 SMALL_LAUNCH_ROWS = 4096  # launches up to this many rows send groups of <= 128 rows to the small kernel
 SPLIT_MAX_ROUNDS = 8      # a row product of this many full rounds of tiles or more is never K-split
+SPLIT_MIN_STEPS = 8       # steps of 64 in a K range: a product of fewer than twice as many is never split
 
 
 @functools.lru_cache(maxsize=None)
@@ -265,20 +266,22 @@ def _device_cus(index: int) -> int:
     return torch.cuda.get_device_properties(index).multi_processor_count
 
 
-def _split_workspace(dev, rows_routed: int = 0, rows_shared: int = 0, tile_cols: int = 0, small: bool = False):
-    """fp32 workspace for the K-split last round of the row products, or
-    (None, 0) when the launch cannot split a tile (the library then runs
-    every tile whole): a decode-sized forward launch whose groups all go to
-    the small-group kernel (small: the product has one; at most 256 routed
-    and 128 shared rows in at most SMALL_LAUNCH_ROWS), or a product of
+def _split_workspace(dev, rows_routed: int, rows_shared: int, depth: int, tile_cols: int, small: bool = False):
+    """fp32 workspace for the K-split tiles of the row products, or (None, 0)
+    when the launch splits none (the library then runs every tile whole): a
+    product of fewer than 2 * SPLIT_MIN_STEPS K steps (depth: its reduction
+    length), a decode-sized forward launch whose groups all go to the
+    small-group kernel (small: the product has one; at most 256 routed and 128
+    shared rows in at most SMALL_LAUNCH_ROWS), or a product of
     SPLIT_MAX_ROUNDS rounds or more (tile_cols: output tiles per 256-row
     block)."""
+    if depth // 64 < 2 * SPLIT_MIN_STEPS:
+        return None, 0
     if small and rows_routed <= 256 and rows_shared <= 128 and rows_routed + rows_shared <= SMALL_LAUNCH_ROWS:
         return None, 0
-    if tile_cols:
-        blocks = -(-rows_routed // 256) + -(-rows_shared // 256)
-        if blocks * tile_cols >= SPLIT_MAX_ROUNDS * _device_cus(dev.index if dev.index is not None else 0):
-            return None, 0
+    blocks = -(-rows_routed // 256) + -(-rows_shared // 256)
+    if blocks * tile_cols >= SPLIT_MAX_ROUNDS * _device_cus(dev.index if dev.index is not None else 0):
+        return None, 0
     lib = _lib.load()
     nbytes = lib.fmoe_split_workspace_bytes()
     return torch.empty(max(nbytes, 16), dtype=torch.uint8, device=dev), nbytes
@@ -293,7 +296,7 @@ def down_fwd(h, offsets, n_experts: int, rows_routed: int, rows_shared: int, w2s
     lib = _lib.load()
     rows, inter = h.shape
     out = torch.empty(rows, dim, dtype=torch.bfloat16, device=h.device)
-    ws, ws_bytes = _split_workspace(h.device, rows_routed, rows_shared, -(-dim // 256), small=True)
+    ws, ws_bytes = _split_workspace(h.device, rows_routed, rows_shared, inter, -(-dim // 256), small=True)
     check(lib.fmoe_down_fwd(_req(h, "h", torch.bfloat16), _req(offsets, "offsets", torch.int32), n_experts,
                             rows_routed, rows_shared, dim, inter, ptr_array([w.data_ptr() for w in w2s]),
                             out.data_ptr(), _ptr(ws), ws_bytes, _stream()),
@@ -348,7 +351,7 @@ def down_bwd_dx(d_out_routed, d_out_shared, offsets, n_experts: int, w2s, ab, in
     if len(w2s) < G:
         raise RuntimeError(f"down_bwd_dx needs {G} weight matrices (got {len(w2s)})")
     d_ab = torch.empty(rows_r + rows_s, 2 * inter, dtype=torch.bfloat16, device=ab.device)
-    ws, ws_bytes = _split_workspace(ab.device, rows_r, rows_s, -(-inter // 256))
+    ws, ws_bytes = _split_workspace(ab.device, rows_r, rows_s, d, -(-inter // 256))
     check(lib.fmoe_down_bwd_dx(_req(d_out_routed, "d_out", torch.bfloat16),
                                _req(d_out_shared, "d_out_shared", torch.bfloat16) if d_out_shared is not None else None,
                                _req(offsets, "offsets", torch.int32), n_experts, rows_r, rows_s, d, inter,
@@ -368,7 +371,7 @@ def gateup_bwd_dx(d_ab, offsets, n_experts: int, rows_routed: int, rows_shared: 
     if len(w1s) < G or len(w3s) < G:
         raise RuntimeError(f"gateup_bwd_dx needs {G} weight matrices of each kind")
     dx_rows = torch.empty(rows, dim, dtype=torch.bfloat16, device=d_ab.device)
-    ws, ws_bytes = _split_workspace(d_ab.device, rows_routed, rows_shared, -(-dim // 256))
+    ws, ws_bytes = _split_workspace(d_ab.device, rows_routed, rows_shared, two_i, -(-dim // 256))
     check(lib.fmoe_gateup_bwd_dx(_req(d_ab, "d_ab", torch.bfloat16), _req(offsets, "offsets", torch.int32),
                                  n_experts, rows_routed, rows_shared, dim, inter,
                                  _weights(w1s[:G], "w1", (inter, dim)), _weights(w3s[:G], "w3", (inter, dim)),

@@ -112,6 +112,20 @@ std::vector<const void*> weight_ptrs(const std::vector<Tensor>& ws, size_t G, co
   return p;
 }
 
+// Bytes of split workspace that a row product of K steps k_steps and tile_cols
+// output tiles per 256-row block can use: none if it runs every tile whole (as
+// _split_workspace of _kernels.py, and launch_rows of the library, have it):
+// fewer than 16 steps, 8 full rounds of tiles or more, or a forward launch
+// (small) whose groups all go to the small-group kernel.
+size_t split_bytes(int64_t rows_routed, int64_t rows_shared, int64_t k_steps, int64_t tile_cols, bool small) {
+  if (k_steps < 16) return 0;
+  if (small && rows_routed <= 256 && rows_shared <= 128 && rows_routed + rows_shared <= 4096) return 0;
+  const size_t bytes = api.fmoe_split_workspace_bytes();
+  const int64_t cus = static_cast<int64_t>(bytes / (256 * 256 * sizeof(float)));  // one partial tile per CU
+  const int64_t blocks = (rows_routed + 255) / 256 + (rows_shared + 255) / 256;
+  return blocks * tile_cols >= 8 * cus ? 0 : bytes;
+}
+
 // One workspace for a pass: its launches run one after the other on one
 // stream, so the largest request serves all of them.
 struct Workspace {
@@ -152,7 +166,8 @@ std::vector<Tensor> forward(const Tensor& x, const Tensor& gate_w, const Tensor&
       throw std::runtime_error("counts_host must be a contiguous pinned int32 CPU tensor of n_experts elements");
     ch = c.data_ptr();
   }
-  const size_t split = api.fmoe_split_workspace_bytes();
+  const size_t split = std::max(split_bytes(rows_r, rows_s, d / 64, (inter + 127) / 128, true),
+                                split_bytes(rows_r, rows_s, inter / 64, (d + 255) / 256, true));
   const size_t rd = api.fmoe_route_and_dispatch_workspace_bytes(T, E, kk);
   const Workspace ws(std::max(split, rd), x);
   check(api.fmoe_route_and_dispatch(xp, gwp, gbp, T, d, E, kk, static_cast<float>(route_scale),
@@ -205,7 +220,8 @@ std::vector<Tensor> backward(const Tensor& dy, const Tensor& x, const Tensor& ga
              *xpp = req(x_perm, "x_perm", bf), *vp = req(v, "topv", at::kFloat);
   const int32_t* off = static_cast<const int32_t*>(offp);
   const int32_t* permp = static_cast<const int32_t*>(pp);
-  const size_t split = api.fmoe_split_workspace_bytes();
+  const size_t split = std::max(split_bytes(rows_r, rows_s, d / 64, (inter + 255) / 256, false),
+                                split_bytes(rows_r, rows_s, 2 * inter / 64, (d + 255) / 256, false));
   const size_t g2 = api.fmoe_weight_grad_workspace_bytes(rows_r, rows_s, E, d, inter);
   const size_t g13 = api.fmoe_weight_grad_workspace_bytes(rows_r, rows_s, E, 2 * inter, d);
   const size_t rb = api.fmoe_router_bwd_workspace_bytes(T, d, E, kk);

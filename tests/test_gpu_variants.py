@@ -222,3 +222,26 @@ def test_gathered_weight_gradient_equals_the_copied_rows(gpu_device, counts, sha
     K.weight_grad(a, sa, x, sb, off, E, rr, shared, m, outs[1], None, torch.float32, b_gather=perm, k=k)
     for want, got in zip(*outs):
         assert torch.equal(want, got)
+
+
+@pytest.mark.parametrize("path", ["native", "wrappers"])
+@pytest.mark.parametrize("T,d,inter,splits", [(300, 256, 448, False), (300, 256, 576, True)])
+def test_split_workspace_only_where_a_launch_can_split(gpu_device, T, d, inter, splits, path):
+    # fewer than 16 K steps of 64 in every product (2 * 448 / 64 = 14): no split,
+    # so no 64 MB of partials; 2 * 576 / 64 = 18 steps in the input gradient
+    cfg = configs.BlockConfig("ws", T, dim=d, inter=inter, n_experts=4, topk=2, n_shared=1, bias="skew")
+    data = configs.make_block(cfg, seed=1)
+    m = DeepSeekMoE(cfg.moe_config())
+    m.load_state_dict(data.state_dict())
+    m = m.to(gpu_device, torch.bfloat16)
+    x = data.x.to(gpu_device, torch.bfloat16).requires_grad_()
+    dy = data.dy.to(gpu_device, torch.bfloat16)
+    K.set_timer({} if path == "wrappers" else None)
+    try:
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        m(x).backward(dy)
+    finally:
+        K.set_timer(None)
+    assert (torch.cuda.max_memory_allocated() - before > 60 << 20) == splits
