@@ -11,8 +11,10 @@ The JSON line also carries:
   roofline      the dominant kernel (largest share of the step) against the
                 MI355X bf16 dense MFMA peak: algorithmic FLOPs per launch over
                 the launch's average duration, timed with HIP events on the
-                stream the kernels run on, inside the timed region (only
-                that entry point carries events there);
+                stream the kernels run on, in steps right after the timed
+                region (which carries none: with events on, the block runs
+                through the per-entry-point wrappers instead of its native
+                launch sequences);
   kernels       the same figures for every entry point of the step: the
                 GEMMs from a short untimed pass with events around every
                 entry point (it also names the dominant one), the
@@ -546,11 +548,10 @@ def main():
     kernels = table_of(full, table_steps, s0.elapsed_time(s1) / 1e3)
     dom = max(kernels, key=lambda n: kernels[n]["share"])
 
-    # Timed region: K steps between two synchronisations.  The dominant entry
-    # point's launches are bracketed by HIP events on the stream they run on
-    # (the roofline figures).  A forward-only (decode-sized) run is host-bound,
-    # where even those events add host time: it is timed bare, and its
-    # roofline comes from the table pass.
+    # Timed region: K steps between two synchronisations, bare: what a user's
+    # program runs.  (With a timer set, the block goes through the wrappers of
+    # the entry points, not its native launch sequences.)  The roofline
+    # figures come from the passes around it.
     if args.graph:
         # Decode as a serving loop runs it: the forward captured once into a
         # HIP graph, each step copies the tokens in and replays it.
@@ -564,8 +565,6 @@ def main():
             graph(xin)
         for _ in range(args.warmup):
             step()
-    timer = {}
-    K.set_timer(None if args.fwd_only else timer, only={dom})
     start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
     torch.cuda.synchronize()
     t0 = time.perf_counter()
@@ -575,7 +574,6 @@ def main():
     end.record()
     torch.cuda.synchronize()
     wall = time.perf_counter() - t0
-    K.set_timer(None)
     gpu_s = start.elapsed_time(end) / 1e3
     elapsed = max(gpu_s, wall)
     tok_s = T * args.steps / elapsed
@@ -596,8 +594,6 @@ def main():
                          frac=round(work / (us / 1e6) / PEAK_BF16_FLOPS, 4))
             kernels[name] = e
         dom = max(kernels, key=lambda n: kernels[n]["share"])
-        timer = {}
-    dk = (table_of(timer, args.steps, elapsed) if timer else kernels)[dom]
     if not args.graph and not args.fwd_only:
         # GEMM pass: as many steps as the table pass, with HIP events around
         # the grouped GEMMs only (each 150 us or longer at C2, so the gaps the
@@ -624,6 +620,7 @@ def main():
                              "bound": "hbm", "achieved_gbs": round(work / (us / 1e6) / 1e9, 1),
                              "frac": round(work / (us / 1e6) / PEAK_HBM_BYTES, 4)}
 
+    dk = kernels[dom]
     bound, work = model[dom]
     avg_s = dk["avg_us"] / 1e6
     traffic = hbm_traffic(cfg.name, dom)
