@@ -256,7 +256,9 @@ def gateup_fwd(x_rows, x_shared, offsets, n_experts: int, w1s, w3s, inter: int, 
     return ab, h
 
 
-SMALL_LAUNCH_ROWS = 4096  # launches up to this many rows send groups of <= 128 rows to the small kernel
+# Launches up to this many rows send groups of <= 128 rows to the small-group kernel, if they have at
+# most 8 routed rows per expert on average or no group can have more than 256.
+SMALL_LAUNCH_ROWS = 4096
 SPLIT_MAX_ROUNDS = 8      # a row product of this many full rounds of tiles or more is never K-split
 SPLIT_MIN_STEPS = 8       # steps of 64 in a K range: a product of fewer than twice as many is never split
 

@@ -149,15 +149,6 @@ __device__ __forceinline__ float fast_sigmoid(float a) {
   return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-a * 1.4426950408889634f));
 }
 
-// Top-k order: a beats b if a is NaN and b is not, or a > b.  Scanning experts
-// in ascending order and replacing only on a strict win keeps ties on the
-// lowest index.
-__device__ __forceinline__ bool score_beats(float a, float b) {
-  const bool an = a != a, bn = b != b;
-  if (an || bn) return an && !bn;
-  return a > b;
-}
-
 // Token of a routed slot, floor(n / k) for 0 <= n < 2^29 and 1 <= k <= 8,
 // without a division: the high half of n * m with m = ceil(2^32 / k).  With
 // m k = 2^32 + e, 0 <= e < k, n m / 2^32 = n / k + n e / (k 2^32); the

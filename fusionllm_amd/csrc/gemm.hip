@@ -247,11 +247,12 @@ __device__ __forceinline__ void swiglu_bwd8(const uint4& dhv, const uint4& av, c
 // to bf16, through the wave's 4 KB of LDS one 16-row slice at a time, read
 // back as 16-byte row segments (64 registers, the accumulators are then
 // free); then the slices' a|b are loaded, computed and stored one after
-// another, each slice's loads in registers of their own, so that the compiler
-// can issue them ahead (with the registers of the slice before: C2 310
-// against 253 us).  Two slices of loads issued up front spill 51 registers
-// beside the main loop's (C2 302 us, C5 1855 against 1500 us).  Row pointers
-// are uniform (scalar registers); a lane adds one offset.
+// another; the slice loop is unrolled and the compiler issues a slice's loads
+// ahead of the stores before it.  The kernel spills 11 registers around this
+// epilogue (256 VGPRs; the main loop has none): 243 us at C2, 1423 at C5.  Two
+// slices of loads issued up front spill 51 (C2 302 us, C5 1855 against 1500 in
+// that session).  Row pointers are uniform (scalar registers); a lane adds
+// one offset.
 __device__ __forceinline__ void down_bwd_full_epilogue(const GemmArgs& args, const f32x4 (&acc)[core::FM][core::FN],
                                                        uint8_t* ep, int el, int64_t grow0, int col0) {
   using namespace core;
@@ -1785,7 +1786,7 @@ extern "C" int fmoe_gateup_bwd_dx(const void* d_ab, const int32_t* offsets, int 
 namespace fmoe {
 // Rows per K chunk of the weight gradient (wgrad_chunks rounds a group to the
 // nearest count).  A work unit is (group, chunk, output tile); the chunk is
-// two thirds of one CU's average share (tiles * rows / 64 K steps over 256
+// two thirds of one CU's average share (tiles * rows / 64 K steps over the
 // CUs), so that skewed groups do not leave a long tail, and at least 768 rows:
 // a split tile costs 256 KB of fp32 partial per chunk, written and read once,
 // about six K steps' time.  Measured (dW2 + dW1|dW3, MI355X): T = 1021, d =
@@ -1803,13 +1804,13 @@ namespace fmoe {
 // 270, T = 6100 460 -> 417, T = 16384 870 -> 850; up to T = 1500 unchanged.
 int64_t wgrad_kc(int64_t rows_routed, int64_t rows_shared, int n_experts, int64_t m_out, int64_t n_out) {
   const int64_t rows = rows_routed + rows_shared;
-  const int64_t tiles = ceil_div(m_out, 256) * ceil_div(n_out, 256);
+  const int64_t tiles = ceil_div(m_out, 256) * ceil_div(n_out, 256), cus = device_cus();
   if (n_experts == 1 && rows_shared == 0) {
     const int64_t n_max = (rows + 384) / 768 < 512 ? (rows + 384) / 768 : 512;
     int64_t best_n = 1, best = 0;
     for (int64_t n = 1; n <= n_max; ++n) {
       const int64_t steps = ceil_div(ceil_div(rows, n), 64) + (n > 1 ? 6 : 0);
-      const int64_t cost = ceil_div(n * tiles, 256) * steps * 25 + (n > 1 ? n * tiles + 75 : 0);
+      const int64_t cost = ceil_div(n * tiles, cus) * steps * 25 + (n > 1 ? n * tiles + 75 : 0);
       if (n == 1 || cost < best) {
         best = cost;
         best_n = n;
@@ -1818,7 +1819,7 @@ int64_t wgrad_kc(int64_t rows_routed, int64_t rows_shared, int n_experts, int64_
     const int64_t kc = ceil_div(rows, best_n);
     return kc < 384 ? 384 : kc;
   }
-  const int64_t kc = (tiles * rows / 384) / 64 * 64;
+  const int64_t kc = (2 * tiles * rows / (3 * cus)) / 64 * 64;
   return kc < 768 ? 768 : kc;
 }
 }  // namespace fmoe

@@ -79,16 +79,6 @@ __device__ __forceinline__ void copy16(uint32_t lds, const void* base, uint32_t 
                : "memory");
 }
 
-// Scalar load of two consecutive ints at a wave-uniform address.  The compiler
-// turns uniform reads issued after the copies (inline assembly that clobbers
-// memory) into vector loads whose vmcnt wait would also wait for every copy in
-// flight; a scalar load is tracked by lgkmcnt instead.
-__device__ __forceinline__ int2 sload2(const int32_t* p) {
-  int2 v;
-  asm volatile("s_load_dwordx2 %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)\n" : "=s"(v) : "s"(p) : "memory");
-  return v;
-}
-
 // One 4-byte-per-lane copy global -> LDS (lane l writes LDS bytes lds + 4 l).
 __device__ __forceinline__ void copy4(uint32_t lds, const void* base, uint32_t voff) {
   asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2\n" ::"s"(lds), "v"(voff), "s"(base) : "memory");
@@ -107,18 +97,13 @@ __device__ __forceinline__ void wait_vm_barrier() {
 // The same, waiting for the LDS reads only.
 __device__ __forceinline__ void wait_lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier\n" ::: "memory"); }
 
-// LDS address of fragment f of one operand: the lane's row (16 f + l % 16 of
-// the wave's block) at chunk (l / 16 + 4 * step half), swizzled.  For rows
-// r = base + 16 f + l % 16 with base % 16 == 0, swzk(r) = l & 7, so every
-// fragment address is x + 2048 f for one per-lane x (the wave's row block and
-// l's swizzle), and the K half is one XOR of 64 (chunk bit 2).
+// LDS address of a lane's fragment 0 of one operand: its row (l % 16 of the
+// wave's block) at chunk l / 16, swizzled.  For rows r = base + 16 f + l % 16
+// with base % 16 == 0, swzk(r) = l & 7, so fragment f is 2048 f further on and
+// the second 32-deep half of the stage is one XOR of 64 (chunk bit 2).
 __device__ __forceinline__ uint32_t frag_base(int row0, int lane) {
   const int t = (lane >> 4) ^ (lane & 7);
   return static_cast<uint32_t>((row0 + (lane & 15)) * RB + (t << 4));
-}
-template <int F, int KX>
-__device__ __forceinline__ uint32_t frag_addr(uint32_t x, uint32_t src) {
-  return (x ^ static_cast<uint32_t>(KX)) + (src + 2048u * F);
 }
 
 // ---- operands read as they lie ([K, N] row-major, N contiguous): the weights

@@ -72,7 +72,7 @@ __device__ __forceinline__ uint32_t row_min(uint32_t v) {
 // Top-k of one token from its scores sc[0 .. E) in LDS: lane l of the token's
 // 16 lanes holds those of experts l, l + 16, ... as ordered keys, and each of
 // the k rounds takes the largest key over the lanes, then the lowest expert
-// that has it (score_beats: NaN first, ties to the lowest index; scores are
+// that has it (NaN first, ties to the lowest index; scores are
 // sigmoids, >= +0, whose bits order as they do).  Lane j < k keeps and writes
 // the j-th choice; the chosen scores are summed in choice order.
 // (Every lane scanning all E scores in each round: 64 experts, top-6, d =
@@ -260,7 +260,7 @@ __global__ __launch_bounds__(kRouterTok / R * kRouterLanes) void router_fwd_kern
   __syncthreads();
 
   // scores: lane j of a group computes experts j, j + 16, ... of its tokens
-  // (in place over the logits), then every lane reads all E of its token
+  // (in place over the logits), which the top-k reads back
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     float* lg = lsh + (grp + r * NG) * EB;

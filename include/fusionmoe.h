@@ -183,8 +183,10 @@ int fmoe_gateup_fwd(const void* x_routed, const int32_t* gather, int gather_k,
 
 /* Workspace of the four row products (fmoe_gateup_fwd, fmoe_down_fwd,
  * fmoe_down_bwd_dx, fmoe_gateup_bwd_dx) for the current device: fp32
- * partials of the tiles of the last, partial round of the persistent grid,
- * which are split along K (up to 4 ranges), summed in range order
+ * partials of the tiles of the last, partial round of the persistent grid
+ * (all tiles, in a launch of fewer tiles than CUs), which are split along K
+ * (up to 8 ranges of at least 8 steps of 64, in products of at least 16
+ * steps and fewer than 8 full rounds), summed in range order
  * (deterministic) and then put through the product's epilogue, with the
  * same rounding points as a whole tile.  Passing no (or a smaller)
  * workspace runs those tiles whole.  Calls that share one workspace must

@@ -1,12 +1,12 @@
 """Check the gfx950 machine code of this build for accesses to registers that a
 memory load has not filled yet (not collected: no test_ prefix).
 
-The GEMM kernels issue their LDS fragment reads from inline assembly and
-wait for them with explicit s_waitcnt instructions, which the compiler does
-not see.  If the compiler ever moved, copied or reused a register that such a
-read is still filling (between the read and the s_waitcnt that covers it),
-the kernel would compute with stale values, or a late read would overwrite a
-live one.  This module disassembles the code objects built here (llvm-objdump
+The GEMM kernels issue their global -> LDS copies and their MFMAs from inline
+assembly, with explicit s_waitcnt instructions and barriers among them; their
+LDS fragment reads are the compiler's, which places the waits for them.  If a
+register that a load is still filling were read, moved, copied or reused
+(between the load and the s_waitcnt that covers it), the kernel would compute
+with stale values, or a late load would overwrite a live one.  This module disassembles the code objects built here (llvm-objdump
 from ROCm) and runs a dataflow pass over each kernel's control-flow graph:
 
 * every LDS instruction (ds_*) and scalar memory load (s_load*, s_buffer_load*)
