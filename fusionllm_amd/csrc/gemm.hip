@@ -248,11 +248,12 @@ __device__ __forceinline__ void swiglu_bwd8(const uint4& dhv, const uint4& av, c
 // back as 16-byte row segments (64 registers, the accumulators are then
 // free); then the slices' a|b are loaded, computed and stored one after
 // another; the slice loop is unrolled and the compiler issues a slice's loads
-// ahead of the stores before it.  The kernel spills 11 registers around this
-// epilogue (256 VGPRs; the main loop has none): 243 us at C2, 1423 at C5.  Two
-// slices of loads issued up front spill 51 (C2 302 us, C5 1855 against 1500 in
-// that session).  Row pointers are uniform (scalar registers); a lane adds
-// one offset.
+// ahead of the stores before it.  The copies' offsets and the fragment
+// addresses of the main loop are formed again after it instead of kept (11
+// registers spilled with them, none without: C2 238 -> 232 us, C5 1401 -> 1372, T
+// = 9001, d = 1024, I = 1536 218 -> 213).  Two slices of loads issued up front
+// spill 51 beside them (C2 302 us, C5 1855 against 1500 in that session).  Row
+// pointers are uniform (scalar registers); a lane adds one offset.
 __device__ __forceinline__ void down_bwd_full_epilogue(const GemmArgs& args, const f32x4 (&acc)[core::FM][core::FN],
                                                        uint8_t* ep, int el, int64_t grow0, int col0) {
   using namespace core;
@@ -377,17 +378,8 @@ __global__ __launch_bounds__(core::NT, 1) void rows_gemm_kernel(const GemmArgs a
   constexpr int NBO = (MODE == GATEUP_FWD) ? 2 : 4;
   uint32_t a_off[4], b_off[NBO];
   const int lda = static_cast<int>(args.lda), ldb = static_cast<int>(args.ldb);
-  auto copy_tile = [&](int ti) __attribute__((always_inline)) {
-    int tile, slot, k0;
-    split_item(sp, nk, b + ti * NP, tile, k0, c_kn, slot);
-    const Tile t = locate_tile(args, map, tiles_n, tile);
+  auto form_offsets = [&](const Tile& t) __attribute__((always_inline)) {
     const bool gathered = GA && t.g < args.E;
-    const uint16_t* A = gathered ? args.a_routed
-                        : (t.g < args.E || args.a_shared == nullptr)
-                            ? args.a_routed + static_cast<int64_t>(t.row_base) * args.lda
-                            : args.a_shared;
-    if (!gathered) A += static_cast<int64_t>(t.tm) * BM * args.lda;
-    c_a = reinterpret_cast<const uint8_t*>(A + k0 * BK);
     const int last_row = min(t.M - t.tm * BM, BM) - 1, n0 = t.tn * TN_COLS;
     // the lane as an opaque value: what follows is formed here, not kept in
     // registers through the main loop
@@ -401,19 +393,10 @@ __global__ __launch_bounds__(core::NT, 1) void rows_gemm_kernel(const GemmArgs a
       const int krow = 4 * w + (l >> 4);
       const int cb = ((((l & 15) >> 1) ^ wsw(krow)) << 1) | (l & 1);
       const int col = 128 * (cb >> 3) + 8 * (cb & 7);  // + 64 u: its column of the tile
-      // GATEUP_BWD: k < inter from w1, else from w3
-      const int kb = k0 * BK;
-      const bool hi = MODE == GATEUP_BWD && kb >= args.inter;
-      c_b0 = reinterpret_cast<const uint8_t*>((hi ? args.b1[t.g] : args.b0[t.g]) +
-                                              static_cast<int64_t>(hi ? kb - args.inter : kb) * args.ldb);
-      c_b1 = reinterpret_cast<const uint8_t*>(args.b1[t.g]);
-      c_ksw = hi ? INT32_MAX : args.inter / BK - k0;
 #pragma unroll
       for (int q = 0; q < 4; ++q)
         b_off[q] = static_cast<uint32_t>((32 * (q & 1) + krow) * ldb + min(n0 + 64 * (q >> 1) + col, args.N - 8)) * 2u;
     } else {
-      c_b0 = reinterpret_cast<const uint8_t*>(args.b0[t.g] + k0 * BK);
-      if constexpr (MODE == GATEUP_FWD) c_b1 = reinterpret_cast<const uint8_t*>(args.b1[t.g] + k0 * BK);
       // GATEUP_FWD: the wave's first 64 B rows are w1 rows, the others the w3 rows of the same h columns
 #pragma unroll
       for (int q = 0; q < NBO; ++q) {
@@ -433,6 +416,31 @@ __global__ __launch_bounds__(core::NT, 1) void rows_gemm_kernel(const GemmArgs a
         a_off[q] = static_cast<uint32_t>(r * lda + dchunk * 8) * 2u;
       }
     }
+  };
+  auto copy_tile = [&](int ti) __attribute__((always_inline)) {
+    int tile, slot, k0;
+    split_item(sp, nk, b + ti * NP, tile, k0, c_kn, slot);
+    const Tile t = locate_tile(args, map, tiles_n, tile);
+    const bool gathered = GA && t.g < args.E;
+    const uint16_t* A = gathered ? args.a_routed
+                        : (t.g < args.E || args.a_shared == nullptr)
+                            ? args.a_routed + static_cast<int64_t>(t.row_base) * args.lda
+                            : args.a_shared;
+    if (!gathered) A += static_cast<int64_t>(t.tm) * BM * args.lda;
+    c_a = reinterpret_cast<const uint8_t*>(A + k0 * BK);
+    if constexpr (BTR) {
+      // GATEUP_BWD: k < inter from w1, else from w3
+      const int kb = k0 * BK;
+      const bool hi = MODE == GATEUP_BWD && kb >= args.inter;
+      c_b0 = reinterpret_cast<const uint8_t*>((hi ? args.b1[t.g] : args.b0[t.g]) +
+                                              static_cast<int64_t>(hi ? kb - args.inter : kb) * args.ldb);
+      c_b1 = reinterpret_cast<const uint8_t*>(args.b1[t.g]);
+      c_ksw = hi ? INT32_MAX : args.inter / BK - k0;
+    } else {
+      c_b0 = reinterpret_cast<const uint8_t*>(args.b0[t.g] + k0 * BK);
+      if constexpr (MODE == GATEUP_FWD) c_b1 = reinterpret_cast<const uint8_t*>(args.b1[t.g] + k0 * BK);
+    }
+    form_offsets(t);
   };
   copy_tile(0);
   // Unit u of step it's stage (two instructions): a stage's units are issued
@@ -701,6 +709,15 @@ __global__ __launch_bounds__(core::NT, 1) void rows_gemm_kernel(const GemmArgs a
 #pragma unroll
       for (int j = 0; j < FN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     asm volatile("s_nop 1" ::: "memory");  // VALU writes -> MFMA reads of the accumulators
+    if constexpr (MODE == DOWN_BWD) {
+      // the copies' offsets and the fragment addresses are formed again: kept
+      // across this epilogue they made it spill 11 registers
+      int tile_, k0_, kn_, slot_;
+      split_item(sp, nk, b + c_ti * NP, tile_, k0_, kn_, slot_);
+      form_offsets(locate_tile(args, map, tiles_n, tile_));
+      xa = frag_base(wm * WTM, el);
+      xb = A_BYTES + tr_base(4 * wn, el);
+    }
     // the next tile's first fragments (after the last tile a harmless re-read)
     read_first(sbase + ((it + 1) & 1) * STAGE);
     if (late && it + 1 < total) barrier();

@@ -451,3 +451,31 @@ def test_build_library_needs_no_torch(monkeypatch):
         monkeypatch.setattr(build.importlib.util, "find_spec", lambda name: spec)
         build.build_library(verbose=False)
         assert len(ran) == n
+
+
+def test_row_products_keep_their_accumulators_in_registers(tmp_path):
+    # The main loops hold 128 accumulator registers beside their fragments and
+    # offsets: a kernel that needs scratch memory pays for it in every tile.
+    # (The gathered weight-gradient variant keeps 4 registers there, outside its
+    # main loop.)
+    import shutil
+    import subprocess
+    from fusionllm_amd import build
+    from tests import isa_check as ic
+    obj = build.BUILD_DIR / "gemm.o"
+    if not obj.exists() or not ic.ROCM_LLVM.exists():
+        pytest.skip("no built objects or no LLVM tools here")
+    shutil.copy(obj, tmp_path / "gemm.o")
+    subprocess.run([str(ic.ROCM_LLVM / "llvm-objdump"), "--offloading", "gemm.o"], check=True, capture_output=True,
+                   cwd=tmp_path)
+    dev = next(p for p in tmp_path.iterdir() if "gfx950" in p.name)
+    notes = subprocess.run([str(ic.ROCM_LLVM / "llvm-readelf"), "--notes", str(dev)], check=True,
+                           capture_output=True, text=True).stdout
+    seen = 0
+    for entry in notes.split("  - .agpr_count:")[1:]:
+        name = re.search(r"\.name:\s+(\S+)", entry).group(1)
+        if "rows_gemm_kernel" in name or "wgrad_tr_kernelILb0E" in name:
+            seen += 1
+            assert re.search(r"\.private_segment_fixed_size:\s*0\s", entry), name
+            assert re.search(r"\.vgpr_spill_count:\s*0\s", entry), name
+    assert seen == 6
