@@ -1534,8 +1534,9 @@ int check_row_product(int n_experts, int64_t rows_routed, int64_t rows_shared, i
 
 // Row counts up to which a launch sends groups of <= kSmallM rows to the
 // small-group kernel (decode-sized batches), if they have at most kSmallAvgRows
-// routed rows per expert, or no group can exceed 2 kSmallM rows; all other
-// launches use the tiled kernel for every group.  Both kernels cost their
+// routed rows per expert, or no group can exceed 2 kSmallM rows, or an operand
+// is not 16-byte aligned (a weight that is a view into a larger buffer); all
+// other launches use the tiled kernel for every group.  Both kernels cost their
 // share when groups of both kinds occur, and the tiled one is the faster from
 // about 8 rows per group: it reads a weight once per 256 rows, the small one
 // once per 16 to 128.  Measured (gate/up + down forward, MI355X, small kernel
@@ -1569,13 +1570,24 @@ inline int small_blocks(int64_t max_rows) {
   return mb <= 1 ? 1 : mb <= 2 ? 2 : (mb <= 4 || MODE == DOWN_FWD) ? 4 : 8;
 }
 
+// Whether the operands of a launch are 16-byte aligned, as the tiled kernel's
+// copies of 16 bytes into LDS expect (the small-group kernel's loads take any
+// address that a bf16 may have).
+template <int MODE>
+bool aligned_operands(const GemmArgs& a, int groups) {
+  bool ok = aligned16(a.a_routed) && aligned16(a.a_shared);
+  for (int g = 0; g < groups; ++g) ok = ok && aligned16(a.b0[g]) && (MODE != GATEUP_FWD || aligned16(a.b1[g]));
+  return ok;
+}
+
 template <int MODE>
 int launch_rows(GemmArgs& a, int64_t rows_routed, int64_t rows_shared, int E, void* stream) {
   constexpr int TN_COLS = (MODE == GATEUP_FWD) ? core::BN / 2 : core::BN;
   const int64_t tiles_n = ceil_div(a.N, TN_COLS);
   constexpr bool kHasSmall = (MODE == GATEUP_FWD || MODE == DOWN_FWD);
   a.small_max = (kHasSmall && rows_routed + rows_shared <= kSmallLaunchRows &&
-                 (rows_routed <= kSmallAvgRows * E || (rows_routed <= 2 * kSmallM && rows_shared <= kSmallM)))
+                 (rows_routed <= kSmallAvgRows * E || (rows_routed <= 2 * kSmallM && rows_shared <= kSmallM) ||
+                  !aligned_operands<MODE>(a, E + (rows_shared > 0 ? 1 : 0))))
                     ? kSmallM
                     : 0;
   // A routed group has at most rows_routed rows: when no group can exceed

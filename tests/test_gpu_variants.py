@@ -245,3 +245,28 @@ def test_split_workspace_only_where_a_launch_can_split(gpu_device, T, d, inter, 
     finally:
         K.set_timer(None)
     assert (torch.cuda.max_memory_allocated() - before > 60 << 20) == splits
+
+
+def test_forward_products_of_weights_at_8_byte_offsets(gpu_device):
+    # Weights that are views into one buffer, 8 bytes past a 16-byte boundary:
+    # 11 rows per expert, which aligned operands send to the tiled kernel, go to
+    # the small-group kernel, whose loads take any such address.
+    D, E, rows, d, I = gpu_device, 40, 11, 256, 128
+    g = torch.Generator().manual_seed(3)
+    off, rr = _groups([rows] * E, D)
+    x, h = _bf(rr, d, g=g).to(D), _bf(rr, I, g=g).to(D)
+    buf = _bf(E * (3 * I * d + 8), g=g, scale=0.05).to(D)
+    w1, w3, w2 = [], [], []
+    for e in range(E):
+        at = e * (3 * I * d + 8) + 4
+        for ws, shape in ((w1, (I, d)), (w3, (I, d)), (w2, (d, I))):
+            ws.append(buf[at:at + I * d].view(shape))
+            assert ws[-1].data_ptr() % 16 == 8
+            at += I * d
+    ab, _ = K.gateup_fwd(x, None, off, E, w1, w3, I)
+    o = K.down_fwd(h, off, E, rr, 0, w2, d)
+    for e in range(E):
+        r = slice(e * rows, (e + 1) * rows)
+        assert _rel(ab[r, :I], x[r].float() @ w1[e].float().t()) < BOUND
+        assert _rel(ab[r, I:], x[r].float() @ w3[e].float().t()) < BOUND
+        assert _rel(o[r], h[r].float() @ w2[e].float().t()) < BOUND
