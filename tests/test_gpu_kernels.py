@@ -322,9 +322,10 @@ def _bf(*shape, scale=1.0, g=None):
 
 @pytest.mark.parametrize("counts,shared,d,I", [
     ([0, 300, 517], 400, 192, 320), ([1, 2, 700], 0, 768, 2048), ([256, 256], 256, 256, 128),
-    # decode-sized launches (groups of <= 128 rows go to the small-group kernel,
-    # built for 1, 2, 4 or 8 blocks of 16 rows from a bound on the group sizes;
-    # with at most 256 routed rows, every group, a larger one as 128-row slabs)
+    # decode-sized launches (with at most 8 routed rows per expert, groups of
+    # <= 128 rows go to the small-group kernel, built for 1, 2, 4 or 8 blocks of
+    # 16 rows from a bound on the group sizes; with at most 256 routed rows,
+    # every group, a larger one as 128-row slabs; [33, 64, ..] is above both)
     ([0, 1], 1, 256, 128), ([1, 0, 0, 1, 0, 0, 0, 0], 1, 768, 2048), ([1, 5, 16, 17], 32, 768, 2048),
     ([33, 64, 100, 128, 7], 128, 192, 320), ([129, 3, 0], 2, 256, 512), ([2], 0, 2048, 1408),
     ([200, 40, 16], 128, 768, 2048), ([0, 256], 0, 192, 320),
@@ -516,7 +517,9 @@ def test_split_tail_matches_whole_tiles(gpu_device):
     range order, then the product's own epilogue) against the same tiles run
     whole.  26000 rows of d=768, I=2048 put every product's tile count above
     the 256-CU grid with a remainder: gate/up 1664 tiles, down 312, down
-    backward 832, gate/up backward 312.  Only the fp32 summation order of the
+    backward 832, gate/up backward 312.  (Products of 12 K steps, gate/up and
+    down backward, run whole either way; test_gpu_variants.py compares them
+    at 16 and more.)  Only the fp32 summation order of the
     split tiles differs: an output agrees with the whole-tile one to a few
     bf16 roundings (one on the sum, up to three more through the SwiGLU
     epilogues, each at most 2^-7 relative), and every row of the first group

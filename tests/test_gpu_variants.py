@@ -20,9 +20,9 @@ def _groups(counts, device):
     return off, sum(counts)
 
 
-# bf16 outputs of fp32 sums of bf16 operands: one rounding (2^-9 relative) and
-# the sums' own error (K 2^-24, below it); rel-L2 bound 4e-3 as for one
-# bf16 rounding of every element.
+# bf16 outputs of fp32 sums of bf16 operands: one rounding (rms 1.5e-3 relative,
+# 2^-9 at most) and the sums' own error (K 2^-24, below it); up to three roundings
+# in a row for h, da and db (rms 2.6e-3): rel-L2 bound 4e-3.
 BOUND = 4e-3
 
 
@@ -31,10 +31,12 @@ def _rel(a, b):
 
 
 @pytest.mark.parametrize("counts,shared,d,I", [
-    ([0, 15, 16, 17], 0, 512, 1024),        # 16 steps: the fewest that split; slices of 16 rows
+    # (each launch has more than 256 routed rows, so that none goes to the small-group kernel)
+    ([0, 15, 16, 17, 300], 0, 512, 1024),   # down: 16 steps, the fewest that split; slices of 16 rows
     ([255, 256, 257, 1], 300, 1024, 576),   # tile edges, columns that do not fill a tile
     ([700, 0, 3, 120], 1000, 64, 1088),     # one K step forward, two ranges of the down product
-    ([130] * 16, 0, 1024, 512),             # 8 to 16 rows per expert and more: the small-group limit
+    ([300, 0, 40, 513], 200, 1024, 1408),   # gate/up and down backward split over ragged groups and an empty one
+    ([130] * 16, 0, 1024, 512),             # one row tile of each group, half full
 ])
 def test_row_products_of_small_launches(gpu_device, counts, shared, d, I):
     D = gpu_device
@@ -47,11 +49,16 @@ def test_row_products_of_small_launches(gpu_device, counts, shared, d, I):
     w1 = [_bf(I, d, g=g, scale=0.05).to(D) for _ in range(G)]
     w3 = [_bf(I, d, g=g, scale=0.05).to(D) for _ in range(G)]
     w2 = [_bf(d, I, g=g, scale=0.05).to(D) for _ in range(G)]
-    ab, _ = K.gateup_fwd(x, xs, off, E, w1, w3, I)
+    dor = _bf(rr, d, g=g).to(D)
+    dos = _bf(shared, d, g=g).to(D) if shared else None
+    abi = _bf(rr + shared, 2 * I, g=g).to(D)
+    ab, hf = K.gateup_fwd(x, xs, off, E, w1, w3, I)
     o = K.down_fwd(h, off, E, rr, shared, w2, d)
+    dd = K.down_bwd_dx(dor, dos, off, E, w2, abi, I)
     dx = K.gateup_bwd_dx(dab, off, E, rr, shared, w1, w3, d)
     bounds = [0, *torch.tensor(counts).cumsum(0).tolist()] + ([rr + shared] if shared else [])
     xa = torch.cat([x, xs]) if shared else x
+    da = torch.cat([dor, dos]) if shared else dor
     for q in range(G):
         r = slice(bounds[q], bounds[q + 1])
         if r.stop == r.start:
@@ -61,14 +68,76 @@ def test_row_products_of_small_launches(gpu_device, counts, shared, d, I):
         assert _rel(ab[r, I:], f(xa[r]) @ f(w3[q]).t()) < BOUND
         assert _rel(o[r], f(h[r]) @ f(w2[q]).t()) < BOUND
         assert _rel(dx[r], f(dab[r, :I]) @ f(w1[q]) + f(dab[r, I:]) @ f(w3[q])) < BOUND
+        # h from the a|b of the same launch; da, db: the SwiGLU's derivative at abi
+        assert _rel(hf[r], torch.nn.functional.silu(f(ab[r, :I])) * f(ab[r, I:])) < BOUND
+        a, b = f(abi[r, :I]), f(abi[r, I:])
+        sg, dh = torch.sigmoid(a), f(da[r]) @ f(w2[q])
+        assert _rel(dd[r, :I], dh * b * sg * (1 + a * (1 - sg))) < BOUND
+        assert _rel(dd[r, I:], dh * a * sg) < BOUND
+
+
+@pytest.mark.parametrize("rows", [512, 513])    # 8 rows for each of 64 experts, and one more: all tiled
+@pytest.mark.parametrize("shared", [0, 85, 200])  # none, small slabs, tiled
+@pytest.mark.parametrize("big", [True, False])  # a group above 128 rows beside small ones; none (512 rows: no tiles at all)
+def test_forward_products_at_the_small_group_limit(gpu_device, rows, shared, big):
+    D, E, d, I = gpu_device, 64, 1024, 1024
+    g = torch.Generator().manual_seed(rows + shared)
+    counts = [130 if big else 127, 128, 1, 0, 0]
+    rest = rows - sum(counts)
+    counts += [rest // 59 + (1 if e < rest % 59 else 0) for e in range(59)]
+    assert sum(counts) == rows and len(counts) == E
+    G = E + (1 if shared else 0)
+    off, rr = _groups(counts, D)
+    x, h = _bf(rr, d, g=g).to(D), _bf(rr + shared, I, g=g).to(D)
+    xs = _bf(shared, d, g=g).to(D) if shared else None
+    gd = torch.Generator(device=D).manual_seed(1)
+    ws = torch.randn(3, G, d, I, generator=gd, device=D, dtype=torch.bfloat16).mul_(0.05)
+    w1, w3, w2 = (list(w.unbind(0)) for w in ws)
+    ab, hf = K.gateup_fwd(x, xs, off, E, w1, w3, I)
+    o = K.down_fwd(h, off, E, rr, shared, w2, d)
+    bounds = [0, *torch.tensor(counts).cumsum(0).tolist()] + ([rr + shared] if shared else [])
+    xa = torch.cat([x, xs]) if shared else x
+    for q in range(G):
+        r = slice(bounds[q], bounds[q + 1])
+        if r.stop == r.start:
+            continue
+        f = lambda t: t.float()
+        assert _rel(ab[r, :I], f(xa[r]) @ f(w1[q]).t()) < BOUND
+        assert _rel(ab[r, I:], f(xa[r]) @ f(w3[q]).t()) < BOUND
+        assert _rel(hf[r], torch.nn.functional.silu(f(ab[r, :I])) * f(ab[r, I:])) < BOUND
+        assert _rel(o[r], f(h[r]) @ f(w2[q]).t()) < BOUND
+
+
+def test_split_tiles_match_whole_tiles_in_every_product(gpu_device):
+    # At 16 K steps and more every product of a launch of fewer tiles than CUs
+    # is split. Only the fp32 summation order differs from the same launch
+    # without a workspace: outputs agree to a few bf16 roundings (one on the
+    # sum, up to three more in the SwiGLU epilogues), and do differ somewhere.
+    from tests.gpu_util import close, rel_l2
+    from tests.test_gpu_kernels import _row_products
+    D, d, I = gpu_device, 1024, 1088
+    g = torch.Generator().manual_seed(11)
+    counts, shared = [1500, 700, 0, 300], 500
+    E, G = 4, 5
+    off, rr = _groups(counts, D)
+    t = lambda *s, scale=1.0: _bf(*s, g=g, scale=scale).to(D)
+    args = (D, t(rr, d), t(shared, d), t(rr, d), t(shared, d), off, E, [t(I, d, scale=.05) for _ in range(G)],
+            [t(I, d, scale=.05) for _ in range(G)], [t(d, I, scale=.05) for _ in range(G)], t(rr + shared, 2 * I),
+            t(rr + shared, I, scale=.3), t(rr + shared, 2 * I, scale=.05))
+    split, whole = _row_products(*args, split=True), _row_products(*args, split=False)
+    for name, a, b in zip(("ab", "h", "out", "d_ab", "dx_rows"), split, whole):
+        close(a, b, rtol=3.2e-2, atol=2e-3)
+        assert rel_l2(a, b.float()) < 2e-3, name
+        assert not torch.equal(a, b), f"{name}: no tile was split"
 
 
 @pytest.mark.parametrize("counts,shared,m,n", [
     ([0, 1, 63, 64, 65], 0, 256, 320),       # groups without rows, one stage and its edges
     ([1151, 1152, 1153, 0], 0, 512, 256),    # one chunk or two (kc = 768: from 1152 rows)
     ([100, 2000], 5000, 64, 704),            # shared group in several chunks, a partial tile
-    ([1151], 0, 320, 256),                   # one group: the chunk count that fills whole rounds
-    ([1152], 0, 320, 256),                   # two chunks from here
+    ([10766, 5], 0, 64, 704),                # 14 chunks of 832 rows: the last one empty, a zero partial
+    ([1216], 0, 320, 256),                   # one group: the chunk count that fills whole rounds, here one
+    ([1217], 0, 320, 256),                   # ... and two from here
     ([5000], 0, 2048, 1536),                 # 48 tiles in five chunks, the last shorter
 ])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
@@ -88,7 +157,7 @@ def test_weight_gradient_chunks(gpu_device, counts, shared, m, n, dtype):
         if A.shape[0] == 0:
             assert not outs[q].any()  # a group without rows: zeros
         else:
-            # fp32: sums of at most 5000 exact products, error about sqrt(rows) 2^-24 per unit
+            # fp32: sums of at most 11000 exact products, error about sqrt(rows) 2^-24 per unit
             assert _rel(outs[q], want) < (BOUND if dtype == torch.bfloat16 else 2e-6)
 
 
@@ -270,3 +339,22 @@ def test_forward_products_of_weights_at_8_byte_offsets(gpu_device):
         assert _rel(ab[r, :I], x[r].float() @ w1[e].float().t()) < BOUND
         assert _rel(ab[r, I:], x[r].float() @ w3[e].float().t()) < BOUND
         assert _rel(o[r], h[r].float() @ w2[e].float().t()) < BOUND
+
+
+@pytest.mark.parametrize("E,k,nans", [(2, 1, [1]), (8, 2, [5]), (17, 3, [16]), (33, 5, [20, 4]), (64, 8, [63, 32, 31])])
+def test_topk_with_nan_experts_among_finite_scores(gpu_device, E, k, nans):
+    # A NaN score beats every finite one; several go to the lowest index first,
+    # then the finite ones in order: torch's stable descending sort.
+    T, d = 50, 64
+    g = torch.Generator().manual_seed(E)
+    x = torch.zeros(T, d).bfloat16()
+    x[:, 0] = 1.0
+    gw = torch.zeros(E, d).bfloat16()
+    gw[:, 0] = torch.randint(-2, 3, (E,), generator=g).bfloat16()
+    gw[nans, 1] = float("nan")  # 0 * NaN: this expert's score is NaN for every token
+    score = gw[:, 0].float()
+    score[nans] = float("nan")
+    idx, _, w, v = K.router_fwd(x.to(gpu_device), gw.to(gpu_device), torch.zeros(E).bfloat16().to(gpu_device), k, 1.0)
+    want = torch.sort(score, descending=True, stable=True).indices[:k]
+    assert torch.equal(idx.cpu().long(), want.expand(T, k))
+    assert torch.equal(torch.isnan(v.cpu()), torch.isnan(score[want]).expand(T, k))
