@@ -386,6 +386,7 @@ def _grad_outputs(outs, name, n_groups, numel, dtype):
     """Addresses of the groups' outputs; the kernel writes numel values of dtype to each."""
     if len(outs) < n_groups:
         raise RuntimeError(f"weight_grad needs {n_groups} outputs in {name} (got {len(outs)})")
+    outs = outs[:n_groups]
     for o in outs:
         _req(o, name, dtype)
         if o.numel() != numel:

@@ -26,13 +26,14 @@
 //   last step the copies repeat the last stage instead of stopping; stores of
 //   an epilogue are waited for like the copies): a few scalar instructions
 //   more in each read phase cost 10-25 % of the loop.
-//   Measured on MI355X, cycles of a 64-deep step (2048 at the MFMA rate): 3270
-//   with one barrier and eight copies per step, both waves of a SIMD in step;
-//   2200 - 2580 in this form (a whole chip on random data then runs at 1.6 -
-//   1.8 GHz, power-limited).  C2 (49152 rows, d = 768, I = 2048): gate/up
-//   forward 355 -> 305 us, down forward 178 -> 148, gate/up dX 304 -> 277; C5
-//   (262144 rows, d = 2048, I = 1408): 2770 -> 2140, 1490 -> 1045, 2560 -> 2140;
-//   outputs bit-identical.
+//   Measured on MI355X, share of a product's cycles in which the MFMA units are
+//   busy (hardware counters), with one barrier and eight copies per step and
+//   both waves of a SIMD in step -> in this form: C2 (49152 rows, d = 768, I =
+//   2048) gate/up forward 0.40 -> 0.50, down forward 0.41 -> 0.58, gate/up dX
+//   0.48 -> 0.57; C5 (229376 rows, d = 2048, I = 1408) 0.45 -> 0.70, 0.41 -> 0.73,
+//   0.49 -> 0.66.  The clock falls with it, at C5 from 2.0 - 2.1 to 1.65 - 1.9 GHz.
+//   Times: C2 355 -> 305 us, 178 -> 148, 304 -> 277; C5 2770 -> 2140, 1490 -> 1045,
+//   2560 -> 2140; outputs bit-identical.
 // * MFMA operands are swapped (srcA = B fragment, srcB = A fragment), so that a
 //   lane's 4 accumulators hold 4 consecutive output columns of one row:
 //   acc[i][j] of lane l = C[16 i + l % 16][16 j + 4 (l / 16) + 0..3].
